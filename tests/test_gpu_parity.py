@@ -331,6 +331,26 @@ def test_grouping_many_clusters_bit_exact(dim, n, clusters, iterations):
     np.testing.assert_array_equal(perm.cpu().numpy(), eperm)
 
 
+@pytest.mark.parametrize("dim,dtype", [(64, torch.float16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("n,clusters", [(256 * 128, 9), (256 * 128 + 1, 9), (512 * 128 - 1, 200)])
+def test_grouping_sorted_update_at_its_tile_chunks(dim, dtype, n, clusters):
+    # The general schedule's update forms the partials of 256 tiles at a time: exactly one full
+    # chunk, one token past it, and two chunks with a partial last tile and clusters that many
+    # tiles do not hold. V is sorted by channel 0, so a cluster's tokens fill some tiles whole
+    # (its longest list) and miss others. Labels, centers and next centers are the oracle's.
+    _print_case("grouping sorted update", dim, dtype, n, clusters)
+    g = torch.Generator().manual_seed(7)
+    v = torch.randn(1, 1, n, dim, generator=g)
+    v[0, 0, :, 0] = v[0, 0, :, 0].sort().values * 8
+    v = v.to(dtype)
+    perm, labels, centers, nxt = vcx.group_values(v.to(DEV), clusters, 2, debug=True, return_centers=True)
+    eperm, elabels, ecenters, enext = o.group_values(bits(v), clusters, 2, dtype_name(dtype), return_next=True)
+    np.testing.assert_array_equal(labels.cpu().numpy(), elabels)
+    np.testing.assert_array_equal(centers.cpu().numpy().view(np.uint32), ecenters.view(np.uint32))
+    np.testing.assert_array_equal(nxt.cpu().numpy().view(np.uint32), enext.view(np.uint32))
+    np.testing.assert_array_equal(perm.cpu().numpy(), eperm)
+
+
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("n,clusters,iterations", [(1, 8, 2), (127, 3, 3), (2049, 8, 2), (5000, 8, 3)])
 def test_grouping_general_schedule_equals_fused(dtype, n, clusters, iterations):
