@@ -233,32 +233,60 @@ __device__ inline float half_wave_max(float v) {
   return max_xor16(v);
 }
 
-// Normalized Sylvester-Hadamard rotation of one row of W = CPT * L values held by L
-// consecutive lanes (lane c of the group holds entries c*CPT .. c*CPT + CPT - 1). Strides
-// 1, 2, 4, ... in order: the in-lane strides first, then lane xor 1, 2, ...; each pair
-// (a, b) with a the lower entry becomes (RN(a + b), RN(a - b)); then every entry is
-// multiplied by norm = RN_f32(1/sqrt(W)). Every lane of the group must take part.
-// Reference: hadamard, src/vc_attention/core.py:79-92; transform_qk_kernel, csrc/kernels.cu:104-123.
-template <int CPT, int L>
-__device__ inline void hadamard_row(float (&x)[CPT], int c, float norm) {
+// Value of lane l ^ M (M in {1, 2, 4, 8}) of the same row of 16 lanes, by DPP moves: quad_perm
+// for 1 and 2, half-row mirror then quad mirror (l ^ 7 ^ 3) for 4, rotation by 8 for 8.
+template <int M>
+__device__ inline float row_xor(float v) {
+  if constexpr (M == 1) return dpp_move<0xB1>(v);
+  else if constexpr (M == 2) return dpp_move<0x4E>(v);
+  else if constexpr (M == 4) return dpp_move<0x1B>(dpp_move<0x141>(v));
+  else return dpp_move<0x128>(v);
+}
+
+// One butterfly stage of the rotation across lanes l and l ^ M: the lower entry becomes
+// RN(a + b), the upper one RN(a - b). The upper lane adds its own entry negated. With eight
+// entries per lane the DPP moves of one entry fill the wait states of another (rotated Q/K
+// quantization at [1,28,37741,128] 259 -> 228 us); with fewer they stall, and distances 4 and 8
+// take the LDS-pipe permute ([1,40,32760,64]: 159 us by DPP, 152 us so).
+template <int M, int CPT>
+__device__ inline void hadamard_lanes(float (&x)[CPT], int c) {
+  const uint32_t flip = (c & M) ? 0x80000000u : 0u;
 #pragma unroll
-  for (int s = 1; s < CPT; s <<= 1)
+  for (int j = 0; j < CPT; ++j)
+    x[j] = __fadd_rn(M >= 4 && CPT < 8 ? __shfl_xor(x[j], M, 64) : row_xor<M>(x[j]),
+                     __uint_as_float(__float_as_uint(x[j]) ^ flip));
+}
+
+// One butterfly stage between a lane's entries j and j + S.
+template <int S, int CPT>
+__device__ inline void hadamard_entries(float (&x)[CPT]) {
 #pragma unroll
-    for (int j = 0; j < CPT; ++j)
-      if (!(j & s)) {
-        const float a = x[j], b = x[j + s];
-        x[j] = __fadd_rn(a, b);
-        x[j + s] = __fsub_rn(a, b);
-      }
-  // Lane xor 1 and 2 stay inside a quad of lanes: a DPP quad_perm move reads the partner
-  // ([1,0,3,2] = 0xB1, [2,3,0,1] = 0x4E) without the LDS-pipe permute of __shfl_xor.
-#pragma unroll
-  for (int m = 1; m < L; m <<= 1)
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) {
-      const float other = m == 1 ? dpp_move<0xB1>(x[j]) : m == 2 ? dpp_move<0x4E>(x[j]) : __shfl_xor(x[j], m, 64);
-      x[j] = (c & m) ? __fsub_rn(other, x[j]) : __fadd_rn(x[j], other);
+  for (int j = 0; j < CPT; ++j)
+    if (!(j & S)) {
+      const float a = x[j], b = x[j + S];
+      x[j] = __fadd_rn(a, b);
+      x[j + S] = __fsub_rn(a, b);
     }
+}
+
+// Normalized Sylvester-Hadamard rotation of one row of W = CPT * L values held by L (at most
+// 16) consecutive lanes. SPLIT = false: lane c of the group holds entries c*CPT .. c*CPT + CPT
+// - 1. SPLIT = true (CPT = 8, L = 16): it holds entries 4c .. 4c + 3 and 64 + 4c .. 64 + 4c + 3,
+// so that a row's binary32 values move in 16-byte pieces of adjacent lanes. Strides 1, 2, 4,
+// ... in order; each pair (a, b) with a the lower entry becomes (RN(a + b), RN(a - b)); then
+// every entry is multiplied by norm = RN_f32(1/sqrt(W)). Every lane of the group must take part.
+// Reference: hadamard, src/vc_attention/core.py:79-92; transform_qk_kernel, csrc/kernels.cu:104-123.
+template <int CPT, int L, bool SPLIT = false>
+__device__ inline void hadamard_row(float (&x)[CPT], int c, float norm) {
+  static_assert(!SPLIT || (CPT == 8 && L == 16), "split rows hold 2 x 4 entries on 16 lanes");
+  if constexpr (CPT > 1) hadamard_entries<1>(x);
+  if constexpr (CPT > 2) hadamard_entries<2>(x);
+  if constexpr (CPT > 4 && !SPLIT) hadamard_entries<4>(x);
+  if constexpr (L > 1) hadamard_lanes<1>(x, c);
+  if constexpr (L > 2) hadamard_lanes<2>(x, c);
+  if constexpr (L > 4) hadamard_lanes<4>(x, c);
+  if constexpr (L > 8) hadamard_lanes<8>(x, c);
+  if constexpr (SPLIT) hadamard_entries<4>(x);
 #pragma unroll
   for (int j = 0; j < CPT; ++j) x[j] = __fmul_rn(x[j], norm);
 }

@@ -202,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void tile_stats_kernel(
 
 // ---------------------------------------------------------------- finalize
 
-// grid (B*H), D threads. km = RN_in(RN_f32(sum over tiles / n)); also the
+// One thread per channel of head bh. km = RN_in(RN_f32(sum over tiles / n)); also the
 // widened value for the K quantizer and, optionally, the caller's km_out.
 // RAW (FP8 block path, vc27): km = RN_f32(sum / n), written to km_f32 and, as binary32,
 // to the caller's km_out.
@@ -239,12 +239,6 @@ __device__ inline void k_mean_body(const double* sums, int64_t tiles, int64_t n,
     km_f32[bh * D + ch] = in_to_f32<DT>(bits);
     if (km_out) static_cast<uint16_t*>(km_out)[bh * D + ch] = static_cast<uint16_t>(bits);
   }
-}
-
-template <int DT, bool RAW = false>
-__global__ void k_mean_kernel(const double* sums, int64_t tiles, int64_t n, int D, float* km_f32,
-                              void* km_out) {
-  k_mean_body<DT, RAW>(sums, tiles, n, D, km_f32, km_out, blockIdx.x, threadIdx.x);
 }
 
 // grid (B*H), D * S threads (S = 1024 / D slices of the tiles). Smoothing off: vs =
@@ -454,6 +448,21 @@ __device__ inline float elem(const void* x, int64_t i) {
   else return in_to_f32<DT>(static_cast<const uint16_t*>(x)[i]);
 }
 
+// Four adjacent elements from element index i (on a four-element boundary), widened.
+template <int DT>
+__device__ inline void load_quad(const void* x, int64_t i, float (&v)[4]) {
+  if constexpr (DT == VCX_FLOAT32) {
+    const float4 q = *reinterpret_cast<const float4*>(static_cast<const float*>(x) + i);
+    v[0] = q.x, v[1] = q.y, v[2] = q.z, v[3] = q.w;
+  } else {
+    const uint2 q = *reinterpret_cast<const uint2*>(static_cast<const uint16_t*>(x) + i);
+    v[0] = in_to_f32<DT>(q.x & 0xffffu), v[1] = in_to_f32<DT>(q.x >> 16);
+    v[2] = in_to_f32<DT>(q.y & 0xffffu), v[3] = in_to_f32<DT>(q.y >> 16);
+  }
+}
+
+constexpr int kPreRows = 4;  // rows per thread of pre_rows_kernel
+
 // grid (tiles, B*H), D threads: binary64 sum of channel d over the tile's keys in key order.
 template <int DT>
 __global__ __launch_bounds__(128) void pre_tile_sum_kernel(const void* x, int64_t H, int64_t n, int64_t sb,
@@ -475,45 +484,105 @@ __global__ __launch_bounds__(128) void pre_tile_sum_kernel(const void* x, int64_
   part[(bh * tiles + t) * D + d] = s;
 }
 
-// grid (ceil(n / RPB), B*H): RPB rows of one head per block; L = min(W, 16) lanes per row
-// with CPT = W / L entries each. out = rotate(x - mean) (mean nullable), [B*H][n][W] binary32.
-template <int DT, int W>
-__global__ __launch_bounds__(kThreads) void pre_rotate_kernel(const void* x, int64_t H, int64_t n, int D,
-                                                              int64_t sb, int64_t sh, int64_t sn,
-                                                              const float* mean, float* out, float norm) {
-  constexpr int L = W < 16 ? W : 16, CPT = W / L, RPB = kThreads / L;
-  const int tid = threadIdx.x, c = tid % L;
-  const int64_t bh = blockIdx.y, r = static_cast<int64_t>(blockIdx.x) * RPB + tid / L;
-  const bool valid = r < n;
-  const int64_t g = bh * n + r;
-  const int64_t off = (bh / H) * sb + (bh % H) * sh + (valid ? r : 0) * sn;
-  float v[CPT];
+// The same sums where every row starts on 8 bytes and D is 64 or 128: grid (ceil(tiles *
+// LT / 64), B*H) one-wave blocks, LT = D / 4 lanes per tile with four adjacent channels each.
+// One 8-byte load (16 for binary32) brings a lane four channels of a key and kBatch keys are
+// in flight, where a thread per channel moves 2 bytes per load ([1,28,37741,128] bf16:
+// 79 us with that, 46 us with this).
+template <int DT, int D>
+__global__ __launch_bounds__(64) void pre_tile_sum_wide_kernel(const void* x, int64_t H, int64_t n, int64_t sb,
+                                                               int64_t sh, int64_t sn, int64_t tiles, double* part) {
+  constexpr int LT = D / 4, kBatch = 16;
+  const int64_t bh = blockIdx.y, t = static_cast<int64_t>(blockIdx.x) * (64 / LT) + threadIdx.x / LT;
+  const int c = threadIdx.x % LT;
+  if (t >= tiles) return;
+  const int64_t off = (bh / H) * sb + (bh % H) * sh + 4 * c;
+  const int64_t r0 = t * kTile, r1 = r0 + kTile < n ? r0 + kTile : n;
+  double s[4] = {0.0, 0.0, 0.0, 0.0};
+  for (int64_t r = r0; r < r1; r += kBatch) {
+    float v[kBatch][4];
 #pragma unroll
-  for (int j = 0; j < CPT; ++j) {
-    const int ch = c * CPT + j;
-    float y = valid && ch < D ? elem<DT>(x, off + ch) : 0.0f;
-    if (mean != nullptr && valid && ch < D) y = __fsub_rn(y, mean[bh * D + ch]);
-    v[j] = y;
-  }
-  hadamard_row<CPT, L>(v, c, norm);
-  if (valid) {
+    for (int i = 0; i < kBatch; ++i) load_quad<DT>(x, off + (r + i < r1 ? r + i : r) * sn, v[i]);
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) out[g * W + c * CPT + j] = v[j];
+    for (int i = 0; i < kBatch; ++i)
+      if (r + i < r1) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) s[j] = __dadd_rn(s[j], static_cast<double>(v[i][j]));
+      }
   }
+  double2* dst = reinterpret_cast<double2*>(part + (bh * tiles + t) * D + 4 * c);
+  dst[0] = make_double2(s[0], s[1]);
+  dst[1] = make_double2(s[2], s[3]);
 }
 
-// Without rotation: out[B*H*n][D] = x - mean (mean nullable), binary32.
-template <int DT>
-__global__ __launch_bounds__(kThreads) void pre_center_kernel(const void* x, int64_t H, int64_t n, int D,
-                                                              int64_t sb, int64_t sh, int64_t sn,
-                                                              const float* mean, float* out, int64_t total) {
-  for (int64_t i = static_cast<int64_t>(blockIdx.x) * kThreads + threadIdx.x; i < total;
-       i += static_cast<int64_t>(gridDim.x) * kThreads) {
-    const int64_t g = i / D, bh = g / n, r = g % n;
-    const int ch = static_cast<int>(i % D);
-    float y = elem<DT>(x, (bh / H) * sb + (bh % H) * sh + r * sn + ch);
-    if (mean != nullptr) y = __fsub_rn(y, mean[bh * D + ch]);
-    out[i] = y;
+// grid (ceil(n / RPB) (+ 1 with KM), B*H): out = x - mean (mean nullable), rotated with ROT,
+// [B*H][n][ROT ? W : D] binary32. L = min(W, 16) lanes hold a row, CPT = W / L entries each (two
+// groups of four at W = 128, see hadamard_row), and a thread takes NR rows of the block's RPB, their
+// loads issued before any is used; the mean's entries are loaded once.
+// WIDE: D = W and every row starts on four elements, so entries move four at a time (8 or 16
+// byte loads, 16-byte stores), without it one by one. The kernel streams: at [1,28,37741,128]
+// bf16 one row and one-entry loads per thread took 230 us for Q and 442 us with the mean, this
+// form 148 and 139 us (5.8 TB/s).
+// Input rows and outputs are touched once here, non-temporally, so that K stays in the
+// memory-side cache between its sums and this pass.
+// KM (Q's launch): blocks (0, bh) form head bh's K mean instead, beside the Q rows.
+template <int DT, int W, bool ROT, bool WIDE, bool KM>
+__global__ __launch_bounds__(kThreads) void pre_rows_kernel(const void* x, int64_t H, int64_t n, int D, int64_t sb,
+                                                            int64_t sh, int64_t sn, const float* mean, float* out,
+                                                            float norm, KMeanArgs kma) {
+  if constexpr (KM) {
+    if (blockIdx.x == 0) {
+      if (static_cast<int>(threadIdx.x) < D)
+        k_mean_body<VCX_BFLOAT16, true>(kma.sums, kma.tiles, kma.n, D, kma.km, nullptr, blockIdx.y, threadIdx.x);
+      return;
+    }
+  }
+  constexpr int L = W < 16 ? W : 16, CPT = W / L, NR = kPreRows, RPB = kThreads / L * NR;
+  constexpr bool SPLIT = W == 128;
+  const int tid = threadIdx.x, c = tid % L;
+  const int64_t bh = blockIdx.y, r0 = static_cast<int64_t>(KM ? blockIdx.x - 1 : blockIdx.x) * RPB + tid / L;
+  const int64_t head = (bh / H) * sb + (bh % H) * sh;
+  auto channel = [&](int j) { return SPLIT ? 4 * c + (j & 3) + 64 * (j >> 2) : c * CPT + j; };
+  float v[NR][CPT];
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    const int64_t r = r0 + i * (kThreads / L), off = head + (r < n ? r : 0) * sn;
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int j = 0; j < CPT; j += 4) load_quad<DT>(x, off + channel(j), reinterpret_cast<float(&)[4]>(v[i][j]));
+    } else {
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) v[i][j] = channel(j) < D ? elem<DT>(x, off + channel(j)) : 0.0f;
+    }
+  }
+  if (mean != nullptr) {
+    float mu[CPT];
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) mu[j] = channel(j) < D ? mean[bh * D + channel(j)] : 0.0f;
+#pragma unroll
+    for (int i = 0; i < NR; ++i)
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) v[i][j] = __fsub_rn(v[i][j], mu[j]);
+  }
+  const int64_t width = ROT ? W : D;
+#pragma unroll
+  for (int i = 0; i < NR; ++i) {
+    if constexpr (ROT) hadamard_row<CPT, L, SPLIT>(v[i], c, norm);
+    const int64_t r = r0 + i * (kThreads / L);
+    if (r >= n) continue;
+    float* dst = out + (bh * n + r) * width;
+    if constexpr (WIDE) {
+#pragma unroll
+      for (int j = 0; j < CPT; j += 4) {
+        typedef float v4f __attribute__((ext_vector_type(4)));
+        __builtin_nontemporal_store(v4f{v[i][j], v[i][j + 1], v[i][j + 2], v[i][j + 3]},
+                                    reinterpret_cast<v4f*>(dst + channel(j)));
+      }
+    } else {
+#pragma unroll
+      for (int j = 0; j < CPT; ++j)
+        if (channel(j) < width) dst[channel(j)] = v[i][j];
+    }
   }
 }
 
@@ -992,49 +1061,65 @@ int preprocess_launch(const void* q, const void* k, int64_t BH, int64_t H, int64
                       int k_smooth, int hadamard, float* q_out, float* k_out, double* part, float* mean,
                       hipStream_t st) {
   const int64_t tiles = cdiv(Nk, kTile);
-  const float* km = nullptr;
+  // rows of four-element pieces: D 64 or 128 and every row on a four-element boundary
+  constexpr int kQuad = DT == VCX_FLOAT32 ? 16 : 8;
+  auto quads = [&](const void* x, int64_t sb, int64_t sh, int64_t sn) {
+    return (D == 64 || D == 128) && aligned(x, kQuad) && sb % 4 == 0 && sh % 4 == 0 && sn % 4 == 0;
+  };
+  const bool q_wide = quads(q, q_sb, q_sh, q_sn) && aligned(q_out, 16);
+  const bool k_rows = quads(k, k_sb, k_sh, k_sn), k_wide = k_rows && aligned(k_out, 16);
+  KMeanArgs kma{};
   if (k_smooth) {
-    pre_tile_sum_kernel<DT><<<dim3(tiles, BH), static_cast<unsigned>(D), 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn,
-                                                                                   part);
+    kma = KMeanArgs{part, tiles, Nk, mean, nullptr};
+    if (k_rows && D == 128)
+      pre_tile_sum_wide_kernel<DT, 128><<<dim3(cdiv(tiles, 2), BH), 64, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, tiles, part);
+    else if (k_rows)
+      pre_tile_sum_wide_kernel<DT, 64><<<dim3(cdiv(tiles, 4), BH), 64, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, tiles, part);
+    else
+      pre_tile_sum_kernel<DT><<<dim3(tiles, BH), static_cast<unsigned>(D), 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, part);
     VCX_LAUNCHED("pre_tile_sum_kernel");
-    k_mean_kernel<VCX_BFLOAT16, true><<<dim3(BH), static_cast<unsigned>(D), 0, st>>>(
-        part, tiles, Nk, static_cast<int>(D), mean, nullptr);
-    VCX_LAUNCHED("k_mean_kernel");
-    km = mean;
-  }
-  if (!hadamard) {
-    const int64_t tq = BH * Nq * D, tk = BH * Nk * D;
-    pre_center_kernel<DT><<<dim3(static_cast<unsigned>(std::min<int64_t>(cdiv(tq, kThreads), 65536))), kThreads, 0,
-                            st>>>(q, H, Nq, static_cast<int>(D), q_sb, q_sh, q_sn, nullptr, q_out, tq);
-    VCX_LAUNCHED("pre_center_kernel<Q>");
-    pre_center_kernel<DT><<<dim3(static_cast<unsigned>(std::min<int64_t>(cdiv(tk, kThreads), 65536))), kThreads, 0,
-                            st>>>(k, H, Nk, static_cast<int>(D), k_sb, k_sh, k_sn, km, k_out, tk);
-    VCX_LAUNCHED("pre_center_kernel<K>");
-    return VCX_OK;
   }
   int W = 1;
   while (W < D) W <<= 1;
   const float norm = static_cast<float>(1.0 / std::sqrt(static_cast<double>(W)));
-  auto run = [&](auto wc) -> int {
-    constexpr int WW = decltype(wc)::value, L = WW < 16 ? WW : 16, RPB = kThreads / L;
-    pre_rotate_kernel<DT, WW><<<dim3(static_cast<unsigned>(cdiv(Nq, RPB)), static_cast<unsigned>(BH)), kThreads, 0,
-                                st>>>(q, H, Nq, static_cast<int>(D), q_sb, q_sh, q_sn, nullptr, q_out, norm);
-    VCX_LAUNCHED("pre_rotate_kernel<Q>");
-    pre_rotate_kernel<DT, WW><<<dim3(static_cast<unsigned>(cdiv(Nk, RPB)), static_cast<unsigned>(BH)), kThreads, 0,
-                                st>>>(k, H, Nk, static_cast<int>(D), k_sb, k_sh, k_sn, km, k_out, norm);
-    VCX_LAUNCHED("pre_rotate_kernel<K>");
+  // Q, with the K mean in its first blocks, then K
+  auto run = [&](auto wc, auto rot) -> int {
+    constexpr int WW = decltype(wc)::value, L = WW < 16 ? WW : 16, RPB = kThreads / L * kPreRows;
+    constexpr bool ROT = decltype(rot)::value;
+    auto rows = [&](auto wide, auto km, const void* x, int64_t n, int64_t sb, int64_t sh, int64_t sn, const float* mu,
+                    float* out) {
+      constexpr bool KM = decltype(km)::value;
+      pre_rows_kernel<DT, WW, ROT, decltype(wide)::value, KM>
+          <<<dim3(static_cast<unsigned>(cdiv(n, RPB) + (KM ? 1 : 0)), static_cast<unsigned>(BH)), kThreads, 0, st>>>(
+              x, H, n, static_cast<int>(D), sb, sh, sn, mu, out, norm, kma);
+    };
+    auto launch = [&](bool wide, auto km, auto... args) {
+      if constexpr (WW == 64 || WW == 128) {
+        if (wide) return rows(std::true_type(), km, args...);
+      }
+      rows(std::false_type(), km, args...);
+    };
+    if (k_smooth) launch(q_wide, std::true_type(), q, Nq, q_sb, q_sh, q_sn, static_cast<const float*>(nullptr), q_out);
+    else launch(q_wide, std::false_type(), q, Nq, q_sb, q_sh, q_sn, static_cast<const float*>(nullptr), q_out);
+    VCX_LAUNCHED("pre_rows_kernel<Q>");
+    launch(k_wide, std::false_type(), k, Nk, k_sb, k_sh, k_sn, static_cast<const float*>(k_smooth ? mean : nullptr),
+           k_out);
+    VCX_LAUNCHED("pre_rows_kernel<K>");
     return VCX_OK;
   };
-  switch (W) {
-    case 1: return run(std::integral_constant<int, 1>());
-    case 2: return run(std::integral_constant<int, 2>());
-    case 4: return run(std::integral_constant<int, 4>());
-    case 8: return run(std::integral_constant<int, 8>());
-    case 16: return run(std::integral_constant<int, 16>());
-    case 32: return run(std::integral_constant<int, 32>());
-    case 64: return run(std::integral_constant<int, 64>());
-    default: return run(std::integral_constant<int, 128>());
-  }
+  auto width = [&](auto rot) -> int {
+    switch (W) {
+      case 1: return run(std::integral_constant<int, 1>(), rot);
+      case 2: return run(std::integral_constant<int, 2>(), rot);
+      case 4: return run(std::integral_constant<int, 4>(), rot);
+      case 8: return run(std::integral_constant<int, 8>(), rot);
+      case 16: return run(std::integral_constant<int, 16>(), rot);
+      case 32: return run(std::integral_constant<int, 32>(), rot);
+      case 64: return run(std::integral_constant<int, 64>(), rot);
+      default: return run(std::integral_constant<int, 128>(), rot);
+    }
+  };
+  return hadamard ? width(std::true_type()) : width(std::false_type());
 }
 }  // namespace
 

@@ -107,6 +107,27 @@ def test_preprocess_qk_bit_exact_and_matrix_oracle(dim, dtype, k_smooth, rotate)
     torch.testing.assert_close(kd.cpu(), k, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("dim,pad", [(64, 0), (64, 2), (128, 0), (128, 4), (128, 3), (96, 0)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("k_smooth,rotate", [(False, True), (True, False), (True, True)])
+def test_preprocess_qk_row_alignments(dim, pad, dtype, k_smooth, rotate):
+    # Rows of dim + pad elements: on four elements (moved four at a time when dim is 64 or 128)
+    # and off them; row counts at the edges of a block's 64 rows and of a 128-key tile, token-
+    # major heads. The last dimension is contiguous, so no copy is made. Bits are the oracle's.
+    _print_case("preprocess_qk rows", dim, pad, dtype, k_smooth, rotate)
+    gen = torch.Generator().manual_seed(21)
+    name = {torch.float32: "float32", torch.bfloat16: "bfloat16"}[dtype]
+    arg = (lambda x: x.numpy()) if dtype == torch.float32 else bits
+    for nq, nk in ((1, 63), (64, 128), (65, 129)):
+        q, k = [torch.randn(2, n, 3, dim + pad, generator=gen).to(dtype) for n in (nq, nk)]
+        qd, kd = [x.to(DEV)[..., :dim].transpose(1, 2) for x in (q, k)]
+        qo, ko = vcx.preprocess_qk(qd, kd, k_smooth, rotate)
+        q, k = [x[..., :dim].transpose(1, 2).contiguous() for x in (q, k)]
+        eq, ek = o.preprocess_qk(arg(q), arg(k), k_smooth=k_smooth, hadamard=rotate, dtype=name)
+        np.testing.assert_array_equal(qo.cpu().numpy(), eq)
+        np.testing.assert_array_equal(ko.cpu().numpy(), ek)
+
+
 def test_preprocess_qk_long_sequence_bit_exact():
     # many tiles: the mean's per-tile then over-tiles order on a 37741-key head
     q, k, _ = make_qkv(1, 2, 1000, 37741, 128, torch.bfloat16, seed=5, kind="outlier")
