@@ -64,11 +64,13 @@ __device__ inline float f16_bits_to_f32(uint32_t b) {
   return static_cast<float>(h);
 }
 
-// IEEE RN-even float -> bfloat16 bits (NaN kept quiet).
+// IEEE RN-even float -> bfloat16 bits (v_cvt_pk_bf16_f32: one instruction where the integer
+// form takes five and a branch around NaN).
 __device__ inline uint32_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return ((u >> 16) | 0x40u) & 0xffffu;
-  return ((u + 0x7fffu + ((u >> 16) & 1u)) >> 16) & 0xffffu;
+  const __bf16 h = static_cast<__bf16>(f);
+  uint16_t s;
+  __builtin_memcpy(&s, &h, 2);
+  return s;
 }
 
 // IEEE RN-even float -> binary16 bits (v_cvt_f16_f32 under the default RNE mode).
@@ -171,9 +173,8 @@ constexpr float kExpB = 119.6500015258789f;
 // Sage INT8 scale and code for one group (quant_per_thread.py:41-44, IEEE division).
 __device__ inline float int8_scale(float amax) { return __fadd_rn(__fdiv_rn(amax, 127.0f), 1e-7f); }
 __device__ inline int int8_code(float x, float s) {
-  float y = __fdiv_rn(x, s);
-  y = __fadd_rn(y, y >= 0.0f ? 0.5f : -0.5f);
-  return static_cast<int>(truncf(y));
+  const float y = __fdiv_rn(x, s);
+  return static_cast<int>(__fadd_rn(y, __builtin_copysignf(0.5f, y)));  // the conversion truncates
 }
 // int8_code(x, s) with the quotient from r = RN(1/s) (one IEEE division per group):
 // q0 = RN(x*r), e = x - q0*s (one FMA, exact unless it underflows), y = RN(q0 + e*r).
@@ -185,9 +186,14 @@ __device__ inline int int8_code(float x, float s) {
 __device__ inline float recip_rn(float s) { return __fdiv_rn(1.0f, s); }
 __device__ inline int int8_code_r(float x, float s, float r) {
   const float q0 = __fmul_rn(x, r);
-  float y = __builtin_fmaf(__builtin_fmaf(-q0, s, x), r, q0);
-  y = __fadd_rn(y, y >= 0.0f ? 0.5f : -0.5f);
-  return static_cast<int>(truncf(y));
+  const float y = __builtin_fmaf(__builtin_fmaf(-q0, s, x), r, q0);
+  return static_cast<int>(__fadd_rn(y, __builtin_copysignf(0.5f, y)));
+}
+// The codes of four values as bytes, the first lowest.
+__device__ inline uint32_t int8_codes4(const float* x, float s, float r) {
+  const uint32_t lo = __builtin_amdgcn_perm(int8_code_r(x[1], s, r), int8_code_r(x[0], s, r), 0x0c0c0400u);
+  const uint32_t hi = __builtin_amdgcn_perm(int8_code_r(x[3], s, r), int8_code_r(x[2], s, r), 0x04000c0cu);
+  return lo | hi;
 }
 
 // ------------------------------------------------------------------ wave helpers

@@ -66,20 +66,6 @@ __device__ inline void load_key_rows_packed(const uint16_t* base, int64_t sn, co
   for (int i = 0; i < NR; ++i) load_row<D>(base, sn, src[i], c, r[i]);
 }
 
-template <int DT, int D, int NR>
-__device__ inline void load_key_rows(const uint16_t* base, int64_t sn, const int64_t* perm, int64_t bh, int64_t n,
-                                     int64_t key0, int c, float (&v)[NR][D / 16]) {
-  constexpr int CPT = D / 16;
-  Row<D> r[NR];
-  load_key_rows_packed<D, NR>(base, sn, perm, bh, n, key0, c, r);
-#pragma unroll
-  for (int i = 0; i < NR; ++i) {
-    const bool valid = key0 + 16 * i < n;
-#pragma unroll
-    for (int j = 0; j < CPT; ++j) v[i][j] = valid ? row_val<DT, D>(r[i], j) : 0.0f;
-  }
-}
-
 // Per-head base pointer of a strided [B,H,N,D] tensor.
 __device__ inline const uint16_t* head_base(const void* x, int64_t bh, int64_t H, int64_t sb, int64_t sh) {
   int64_t b = bh / H, h = bh % H;
@@ -351,12 +337,7 @@ __global__ __launch_bounds__(kThreads) void quant_q_kernel(const void* q, int64_
     if (row < n) {
       uint32_t packed[CPT / 4];
 #pragma unroll
-      for (int j = 0; j < CPT / 4; ++j) {
-        uint32_t wv = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) wv |= (static_cast<uint32_t>(int8_code_r(x[4 * j + e], s, rs)) & 0xffu) << (8 * e);
-        packed[j] = wv;
-      }
+      for (int j = 0; j < CPT / 4; ++j) packed[j] = int8_codes4(&x[4 * j], s, rs);
       int8_t* dst = q8 + (bh * n + row) * D + c * CPT;
       store_payload_nt<CPT>(dst, packed);
     }
@@ -606,14 +587,16 @@ __global__ __launch_bounds__(kThreads) void quant_k_kernel(const void* k, int64_
   float mean[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) mean[j] = km[bh * D + c * CPT + j];
+  Row<D> rows[8];
+  load_key_rows_packed<D, 8>(base, sn, perm, bh, n, tile * kTile + kk, c, rows);
   float v[8][CPT];
-  load_key_rows<DT, D, 8>(base, sn, perm, bh, n, tile * kTile + kk, c, v);
   float amax = 0.0f;
 #pragma unroll
   for (int i = 0; i < 8; ++i) {
-    const bool valid = tile * kTile + kk + 16 * i < n;
+    const uint32_t keep = tile * kTile + kk + 16 * i < n ? ~0u : 0u;  // keys past n read as zero
 #pragma unroll
-    for (int j = 0; j < CPT; ++j) v[i][j] = valid ? round_in<DT>(__fsub_rn(v[i][j], mean[j])) : 0.0f;
+    for (int j = 0; j < CPT; ++j)
+      v[i][j] = __uint_as_float(__float_as_uint(round_in<DT>(__fsub_rn(row_val<DT, D>(rows[i], j), mean[j]))) & keep);
     if constexpr (ROT) hadamard_row<CPT, 16>(v[i], c, norm);
 #pragma unroll
     for (int j = 0; j < CPT; ++j) amax = fmaxf(amax, fabsf(v[i][j]));
@@ -631,12 +614,7 @@ __global__ __launch_bounds__(kThreads) void quant_k_kernel(const void* k, int64_
     if (key >= n) continue;
     uint32_t packed[CPT / 4];
 #pragma unroll
-    for (int j = 0; j < CPT / 4; ++j) {
-      uint32_t wv = 0;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) wv |= (static_cast<uint32_t>(int8_code_r(v[i][4 * j + e], s, rs)) & 0xffu) << (8 * e);
-      packed[j] = wv;
-    }
+    for (int j = 0; j < CPT / 4; ++j) packed[j] = int8_codes4(&v[i][4 * j], s, rs);
     int8_t* dst = k8 + (bh * n + key) * D + c * CPT;
     store_payload_nt<CPT>(dst, packed);
   }
