@@ -19,7 +19,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "lib" / "libvcx.so"
-SOURCES = ["vcx_abi.hip", "vcx_prep.hip", "vcx_group.hip", "vcx_attn.hip"]
+SOURCES = ["vcx_abi.hip", "vcx_prep.hip", "vcx_group.hip", "vcx_attn.hip", "vcx_attn_piece.hip"]
 
 
 def hipcc() -> str:
@@ -52,7 +52,7 @@ def build(verbose: bool = False) -> Path:
                 print(msg)
         return obj
 
-    with cf.ThreadPoolExecutor(max_workers=min(4, len(SOURCES))) as pool:
+    with cf.ThreadPoolExecutor(max_workers=len(SOURCES)) as pool:
         objs = list(pool.map(compile_one, SOURCES))
     LIB.parent.mkdir(exist_ok=True)
     tmp = LIB.with_suffix(".so.tmp%d" % os.getpid())
