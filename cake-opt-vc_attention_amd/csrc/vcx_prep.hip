@@ -747,6 +747,38 @@ __global__ void convert_probe_kernel(const float* x, uint8_t* u8, uint8_t* f8, i
   f8[i] = static_cast<uint8_t>(e4m3_sat(x[i]));
 }
 
+// Every block writes one word: whether any of its elements has all exponent bits set. Per 16-bit
+// element the exponent field plus its lowest bit carries into the sign position exactly then.
+// VCX_FINITE_BLOCKS blocks, 16-byte pieces dealt to the threads in order, four in flight. One
+// read of the inputs and one word per block to fetch: three torch.isfinite(x).all() took five
+// elementwise passes, a reduction and a wait each (three [1,7,37741,128] bf16 inputs, host wait
+// included: 500 us, this 55 us).
+struct FiniteArgs {
+  const uint4* p[3];
+  int64_t n[3];  // 16-byte pieces
+};
+__global__ __launch_bounds__(256) void finite_kernel(FiniteArgs a, uint32_t mask, uint32_t step, int32_t* out) {
+  constexpr int kBatch = 4;
+  uint32_t bad = 0;
+  const int64_t stride = static_cast<int64_t>(gridDim.x) * blockDim.x;
+#pragma unroll
+  for (int t = 0; t < 3; ++t) {
+    for (int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x; i < a.n[t]; i += kBatch * stride) {
+      uint4 v[kBatch];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) v[b] = a.p[t][i + b * stride < a.n[t] ? i + b * stride : i];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b) {
+        const uint32_t w[4] = {v[b].x, v[b].y, v[b].z, v[b].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) bad |= (w[e] & mask) + step;
+      }
+    }
+  }
+  const bool any = __syncthreads_or((bad & 0x80008000u) != 0);
+  if (threadIdx.x == 0) out[blockIdx.x] = any ? 1 : 0;
+}
+
 // ---------------------------------------------------------------- host helpers
 
 struct Strided {
@@ -1030,6 +1062,25 @@ extern "C" int vcx_convert_probe(const float* x, uint8_t* u8, uint8_t* f8, int64
   convert_probe_kernel<<<cdiv(n, 256), 256, 0, static_cast<hipStream_t>(stream)>>>(x, u8, f8, n);
   VCX_LAUNCHED("convert_probe_kernel");
   return VCX_OK;
+}
+
+extern "C" int vcx_check_finite(const void* a, int64_t na, const void* b, int64_t nb, const void* c, int64_t nc,
+                                int dtype, int32_t* out, void* stream) {
+  VCX_REQUIRE(dtype == VCX_FLOAT16 || dtype == VCX_BFLOAT16, "dtype must be float16 or bfloat16");
+  VCX_REQUIRE(out != nullptr && aligned(out, 4), "out must be non-null and 4-byte aligned");
+  const void* p[3] = {a, b, c};
+  const int64_t n[3] = {na, nb, nc};
+  FiniteArgs args{};
+  for (int t = 0; t < 3; ++t) {
+    VCX_REQUIRE(n[t] >= 0 && n[t] % 8 == 0 && (n[t] == 0 || (p[t] != nullptr && aligned(p[t], 16))),
+                "inputs must be 16-byte aligned with a multiple of 8 elements");
+    args.p[t] = static_cast<const uint4*>(p[t]);
+    args.n[t] = n[t] / 8;
+  }
+  const uint32_t mask = dtype == VCX_BFLOAT16 ? 0x7f807f80u : 0x7c007c00u;
+  const uint32_t step = dtype == VCX_BFLOAT16 ? 0x00800080u : 0x04000400u;
+  finite_kernel<<<VCX_FINITE_BLOCKS, 256, 0, static_cast<hipStream_t>(stream)>>>(args, mask, step, out);
+  return check_launch("finite_kernel");
 }
 
 namespace {

@@ -166,6 +166,14 @@ def _hip_grouping(cfg):
                                                return_centers=True)
 
 
+def _all_finite(q, k, v):
+    if q.device.type != "cuda":
+        return all(bool(torch.isfinite(x).all()) for x in (q, k, v))
+    import vcx
+
+    return vcx.all_finite(q, k, v)
+
+
 def _validate(q, k, v, causal, mask):
     if causal:
         raise ValueError("This experiment does not support causal attention")
@@ -183,7 +191,7 @@ def _validate(q, k, v, causal, mask):
         raise ValueError("Q/K/V must have the same device and dtype")
     if q.dtype not in (torch.float16, torch.bfloat16, torch.float32):
         raise ValueError("Inputs must be FP16/BF16/FP32 before quantization")
-    if not all(bool(torch.isfinite(x).all()) for x in (q, k, v)):
+    if not _all_finite(q, k, v):
         raise ValueError("Q/K/V must be finite")
 
 

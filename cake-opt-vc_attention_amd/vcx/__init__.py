@@ -68,6 +68,8 @@ def _declare(L):
     L.vcx_attention_fwd_fp8.restype = i32
     L.vcx_attention_fwd_fp8.argtypes = [P, P, P, P, P, P, i64, i64, i64, i64, i64, i32, f32, i32,
                                         P, i64, i64, i64, P, i64, i64, P]
+    L.vcx_check_finite.restype = i32
+    L.vcx_check_finite.argtypes = [P, i64, P, i64, P, i64, i32, P, P]
     L.vcx_expcast_codes.restype = i32
     L.vcx_expcast_codes.argtypes = [P, P, i64, P]
     L.vcx_fp8_exp2_codes.restype = i32
@@ -85,7 +87,7 @@ def _declare(L):
 EXPORTED = ("vcx_abi_version", "vcx_last_error", "vcx_value_token", "vcx_workspace_bytes",
             "vcx_group_values", "vcx_prepare_qk_int8", "vcx_prepare_qk_int8_noalloc", "vcx_prepare_qk_int8_rotated",
             "vcx_preprocess_qk",
-            "vcx_prepare_qk_fp8", "vcx_prepare_v_fp8", "vcx_attention_fwd", "vcx_attention_fwd_fp8",
+            "vcx_prepare_qk_fp8", "vcx_prepare_v_fp8", "vcx_attention_fwd", "vcx_attention_fwd_fp8", "vcx_check_finite",
             "vcx_expcast_codes", "vcx_fp8_exp2_codes", "vcx_convert_probe", "vcx_kernel_resources", "vcx_kernel_resources_mode",
             "vcx_kernel_resources_fp8",
             "vcx_clock_probe")
@@ -447,6 +449,27 @@ def forward_fp8(q8, k8, v8, qs, ks, vs, expcast: bool, output_type: int, scale: 
                                        _stream(dev)),
            "vcx_attention_fwd_fp8")
     return (out, pd) if p_rows is not None else out
+
+
+FINITE_BLOCKS = 1024  # VCX_FINITE_BLOCKS
+
+
+def _dense(x) -> bool:
+    """Whether x's elements fill one aligned run of memory (in [B,H,N,D] or [B,N,H,D] order)."""
+    return x.numel() % 8 == 0 and x.data_ptr() % 16 == 0 and (x.is_contiguous() or x.transpose(1, 2).is_contiguous())
+
+
+@_device_call
+def all_finite(q, k, v) -> bool:
+    """Whether three four-dimensional GPU tensors of one dtype hold no NaN or infinity (waits
+    for the answer): one pass over fp16/bf16 tensors that fill their memory, else torch."""
+    if q.dtype not in _DTYPE or not (_dense(q) and _dense(k) and _dense(v)):
+        return all(bool(torch.isfinite(x).all()) for x in (q, k, v))
+    dev = _require_device(q, k, v)
+    out = torch.empty(FINITE_BLOCKS, dtype=torch.int32, device=dev)
+    _check(lib().vcx_check_finite(_ptr(q), q.numel(), _ptr(k), k.numel(), _ptr(v), v.numel(), _DTYPE[q.dtype],
+                                  _ptr(out), _stream(dev)), "vcx_check_finite")
+    return not bool(out.cpu().any())
 
 
 @_device_call

@@ -39,6 +39,7 @@ extern "C" {
 
 #define VCX_ABI_VERSION 3
 #define VCX_CLOCK_PROBE_BLOCKS 8
+#define VCX_FINITE_BLOCKS 1024
 #define VCX_NOALLOC_SCRATCH_BYTES (32u << 20) /* scratch of vcx_prepare_qk_int8_noalloc, per GPU */
 
 enum vcx_status {
@@ -220,6 +221,13 @@ int vcx_attention_fwd_fp8(const uint8_t* q8, const uint8_t* k8, const uint8_t* v
                           int64_t Nk, int64_t D, int expcast, float sm_scale, int out_dtype,
                           void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn, uint8_t* p_dump,
                           int64_t p_row_begin, int64_t p_row_end, void* stream);
+
+/* Whether up to three fp16/bf16 arrays (n elements, a multiple of 8, 16-byte aligned; 0 = none)
+ * hold a NaN or an infinity: out[0..VCX_FINITE_BLOCKS) (device int32) receives words that are
+ * all 0 when every element is finite. Replaces the three torch.isfinite(x).all() of
+ * src/vc_attention/core.py's input checks by one pass. */
+int vcx_check_finite(const void* a, int64_t na, const void* b, int64_t nb, const void* c, int64_t nc,
+                     int dtype, int32_t* out, void* stream);
 
 /* ExpCast byte probe: y[i] = clamp(RNE(fmaf(x[i], 11.54156, 119.65)), 0, 120).
  * Replaces _vc_sm90.expcast_codes (third_party/sageattention_local/csrc/vc/preprocess.cu:170-179). */
