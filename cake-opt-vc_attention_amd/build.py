@@ -19,7 +19,7 @@ from pathlib import Path
 HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 LIB = HERE / "lib" / "libvcx.so"
-SOURCES = ["vcx_abi.hip", "vcx_prep.hip", "vcx_group.hip", "vcx_attn.hip", "vcx_attn_piece.hip"]
+SOURCES = ["vcx_abi.hip", "vcx_call.hip", "vcx_prep.hip", "vcx_group.hip", "vcx_attn.hip", "vcx_attn_piece.hip"]
 
 
 def hipcc() -> str:

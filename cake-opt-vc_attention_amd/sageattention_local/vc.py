@@ -24,6 +24,7 @@ Differences a caller can observe, all deliberate:
   binary64 where an E4M3 rounding midpoint lies within two ulps), so the bytes
   are exact; the row mass sums the unrounded exp2 values.
 """
+import functools
 import math
 
 import torch
@@ -107,10 +108,15 @@ def validate_inputs(q, k, v, tensor_layout, is_causal, return_lse, expcast, v_sm
         raise ValueError("Sage VC requires D=64/128")
 
 
+@functools.lru_cache(maxsize=64)
+def _arch(index):
+    return getattr(torch.cuda.get_device_properties(index), "gcnArchName", "")
+
+
 def _require_gfx950(device):
     if device.type != "cuda" or not torch.cuda.is_available():
         raise ValueError("Sage VC requires an MI355X (gfx950) GPU; no CPU/reference fallback")
-    arch = getattr(torch.cuda.get_device_properties(device), "gcnArchName", "")
+    arch = _arch(device.index)
     if not arch.startswith("gfx950"):
         raise ValueError(f"Sage VC requires gfx950 (MI355X), found {arch or 'unknown'}; no fallback")
 
@@ -152,6 +158,14 @@ def prepare(q, k, v, *, expcast=True, v_smooth=True, clusters=8, iterations=2, s
 AFFINE_MODES = ("optimized", "vc15", "vc14", "vc13_overlap", "vc13_serial", "vc12")
 
 
+def _encode(expcast, block_values, kernel_mode):
+    """Probability path of a mode: 2 folded, 1 unfused ExpCast, 0 the control path."""
+    if not expcast:
+        return 0
+    mode = "vc15" if kernel_mode in SAGE_LAYOUT_MODES else kernel_mode
+    return 2 if not block_values and mode in AFFINE_MODES else 1
+
+
 def forward_prepared(state, *, kernel_mode="optimized", out=None):
     """Fused kernel on a prepared state (reference vc.py:173-197)."""
     channel = not (state["block_values"] and state["vs"].ndim == 4)
@@ -159,8 +173,7 @@ def forward_prepared(state, *, kernel_mode="optimized", out=None):
                 expcast=state["expcast"], dim=state["q"].shape[-1], v_scale_mode="channel" if channel else "block")
     if kernel_mode in UNIFIED_MODES and state["vs"].ndim != 3:
         raise ValueError("vc31/vc32 require per-channel V scale")
-    mode = "vc15" if kernel_mode in SAGE_LAYOUT_MODES else kernel_mode
-    affine = bool(state["expcast"]) and not state["block_values"] and mode in AFFINE_MODES
+    affine = _encode(state["expcast"], state["block_values"], kernel_mode) == 2
     return _extension().forward(state["q"], state["k"], state["v"], state["qs"], state["ks"], state["vs"],
                                 state["means"], state["expcast"], state["block_values"], state["output_type"],
                                 state["scale"], channel_scale=channel, affine=affine, out=out)
@@ -186,19 +199,14 @@ def sageattn_vc(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, re
     validate_inputs(q, k, v, tensor_layout, is_causal, return_lse, expcast, v_smooth, clusters, iterations)
     _require_gfx950(q.device)
     _check_scale(sm_scale)
-    with torch.cuda.device(q.device):
-        if tensor_layout == "NHD":
-            q, k, v = (x.transpose(1, 2) for x in (q, k, v))  # strided HND views, no copy
-            B, H, N, D = q.shape
-            out_nhd = torch.empty((B, N, H, D), dtype=q.dtype, device=q.device)
-            out = out_nhd.transpose(1, 2)
-        else:
-            out_nhd = None
-            out = None
-        state = prepare(q, k, v, expcast=expcast, v_smooth=v_smooth, clusters=clusters, iterations=iterations,
-                        sm_scale=sm_scale, v_scale_mode=v_scale_mode, grouping_mode=grouping_mode)
-        result = forward_prepared(state, kernel_mode=kernel_mode, out=out)
-        return out_nhd if out_nhd is not None else result
+    out = result = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    if tensor_layout == "NHD":
+        q, k, v, out = (x.transpose(1, 2) for x in (q, k, v, out))  # strided HND views, no copy
+    _extension().attention_call(q, k, v, out, expcast=_encode(expcast, v_smooth, kernel_mode), smooth=v_smooth,
+                                channel_scale=v_scale_mode == "channel", clusters=clusters, iterations=iterations,
+                                legacy=grouping_mode == "legacy",
+                                scale=q.shape[-1] ** -0.5 if sm_scale is None else sm_scale)
+    return result
 
 
 # The reference's kernel_resources names (vc_sm90.cu:801-808,1123-1213 and vc.py:113-118), each

@@ -53,18 +53,14 @@ def sageattn_vc_fp8(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None
     validate_inputs(q, k, v, tensor_layout, is_causal, return_lse, expcast, False, 8, 2)
     _require_gfx950(q.device)
     _check_scale(sm_scale)
-    if sm_scale is not None and torch.tensor(sm_scale, dtype=torch.float32).item() == 0:
+    if sm_scale is not None and torch.tensor(sm_scale, dtype=torch.float32, device="cpu").item() == 0:
         raise ValueError("sm_scale must be positive and finite FP32")
-    with torch.cuda.device(q.device):
-        if tensor_layout == "NHD":
-            q, k, v = (x.transpose(1, 2) for x in (q, k, v))  # strided HND views, no copy
-            B, H, N, D = q.shape
-            out_nhd = torch.empty((B, N, H, D), dtype=q.dtype, device=q.device)
-            out = out_nhd.transpose(1, 2)
-        else:
-            out_nhd = out = None
-        result = forward_prepared(prepare(q, k, v, expcast=expcast, sm_scale=sm_scale), out=out)
-        return out_nhd if out_nhd is not None else result
+    out = result = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    if tensor_layout == "NHD":
+        q, k, v, out = (x.transpose(1, 2) for x in (q, k, v, out))  # strided HND views, no copy
+    _extension().attention_call(q, k, v, out, qk_fp8=True, expcast=2 if expcast else 0, smooth=False,
+                                scale=q.shape[-1] ** -0.5 if sm_scale is None else sm_scale)
+    return result
 
 
 def fp8_kernel_resources(output_type=1, dim=128):

@@ -226,11 +226,10 @@ def attention(q, k, v, config=None, *, cache=None, step=0, total_steps=1, reques
                                          layer_id=layer_id)
     import vcx
 
-    q8, qs, k8, ks, km = vcx.prepare_qk(q, k, pi, hadamard=cfg.qk_hadamard)
-    v8, vs, means = vcx.prepare_v(v, pi, smooth=active, channel_scale=True)
     # The ExpCast encode of the reference's default kernel mode: folded without block values.
-    out = vcx.forward(q8, k8, v8, qs, ks, vs, means, cfg.expcast, active, 0 if q.dtype == torch.float16 else 1,
-                      scale, affine=cfg.expcast and not active)
+    out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
+    vcx.attention_call(q, k, v, out, perm=pi, rotate=cfg.qk_hadamard,
+                       expcast=(1 if active else 2) if cfg.expcast else 0, smooth=active, scale=scale)
     return out, {
         "backend": "hip",
         "smoothing_active": active,

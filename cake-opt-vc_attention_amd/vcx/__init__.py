@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import itertools
+import struct
 from pathlib import Path
 
 import torch
@@ -68,6 +69,10 @@ def _declare(L):
     L.vcx_attention_fwd_fp8.restype = i32
     L.vcx_attention_fwd_fp8.argtypes = [P, P, P, P, P, P, i64, i64, i64, i64, i64, i32, f32, i32,
                                         P, i64, i64, i64, P, i64, i64, P]
+    L.vcx_attention_call.restype = i32
+    L.vcx_attention_call.argtypes = [ctypes.c_char_p, P]
+    L.vcx_attention_call_bytes.restype = i32
+    L.vcx_attention_call_bytes.argtypes = [ctypes.c_char_p, ctypes.POINTER(ctypes.c_size_t)]
     L.vcx_check_finite.restype = i32
     L.vcx_check_finite.argtypes = [P, i64, P, i64, P, i64, i32, P, P]
     L.vcx_expcast_codes.restype = i32
@@ -87,7 +92,7 @@ def _declare(L):
 EXPORTED = ("vcx_abi_version", "vcx_last_error", "vcx_value_token", "vcx_workspace_bytes",
             "vcx_group_values", "vcx_prepare_qk_int8", "vcx_prepare_qk_int8_noalloc", "vcx_prepare_qk_int8_rotated",
             "vcx_preprocess_qk",
-            "vcx_prepare_qk_fp8", "vcx_prepare_v_fp8", "vcx_attention_fwd", "vcx_attention_fwd_fp8", "vcx_check_finite",
+            "vcx_prepare_qk_fp8", "vcx_prepare_v_fp8", "vcx_attention_fwd", "vcx_attention_fwd_fp8", "vcx_attention_call", "vcx_attention_call_bytes", "vcx_check_finite",
             "vcx_expcast_codes", "vcx_fp8_exp2_codes", "vcx_convert_probe", "vcx_kernel_resources", "vcx_kernel_resources_mode",
             "vcx_kernel_resources_fp8",
             "vcx_clock_probe")
@@ -449,6 +454,52 @@ def forward_fp8(q8, k8, v8, qs, ks, vs, expcast: bool, output_type: int, scale: 
                                        _stream(dev)),
            "vcx_attention_fwd_fp8")
     return (out, pd) if p_rows is not None else out
+
+
+# struct vcx_call (include/vcx.h): pointers, sizes, strides, options, the softmax scale
+_CALL = struct.Struct("@7q 5q 12q 9q d")
+
+
+@functools.lru_cache(maxsize=256)
+def _call_bytes(shape, options, own_perm: bool) -> int:
+    """Workspace of one vcx_attention_call (a function of the shape and the options alone)."""
+    out = ctypes.c_size_t(0)
+    call = _CALL.pack(0, 0, 0, 0, 0 if own_perm else 1, 0, 0, *shape, *(0,) * 12, *options, 1.0)
+    _check(lib().vcx_attention_call_bytes(call, ctypes.byref(out)), "vcx_attention_call_bytes")
+    return max(out.value, 256)
+
+
+def attention_call(q, k, v, out, *, perm=None, qk_fp8: bool = False, rotate: bool = False, expcast: int, smooth: bool,
+                   channel_scale: bool = True, clusters: int = 8, iterations: int = 2, legacy: bool = False,
+                   scale: float):
+    """One call from [B,H,N,D] Q/K/V to `out` (same dtype and device, [B,H,Nq,D] strides):
+    grouping (smooth without perm), preparation and the fused kernel, on one workspace of the
+    current stream. expcast: 2 folded, 1 unfused ExpCast, 0 the control probabilities. Results
+    are those of group_values, prepare_qk(_fp8), prepare_v and forward(_fp8)."""
+    B, H, Nq, D = q.shape
+    Nk = k.shape[2]
+    qs, ks, vs, os = q.stride(), k.stride(), v.stride(), out.stride()
+    if qs[3] != 1 or ks[3] != 1 or vs[3] != 1 or os[3] != 1:
+        raise VcxError("expected [B,H,N,D] with a contiguous last dimension")
+    dev = _require_device(q, k, v, out, perm)
+    if perm is not None and (perm.dtype != torch.int64 or tuple(perm.shape) != (B, H, Nk) or not perm.is_contiguous()):
+        raise VcxError("perm must be contiguous int64 [B,H,Nk]")
+    shape = (B, H, Nq, Nk, D)
+    options = (_DTYPE[q.dtype], int(qk_fp8), int(rotate), expcast, int(smooth), int(channel_scale), clusters,
+               iterations, GROUP_GENERAL if legacy else GROUP_AUTO)
+    size = _call_bytes(shape, options, perm is None)
+    if torch.cuda.current_device() != dev.index:
+        with torch.cuda.device(dev):
+            return _run_call(q, k, v, out, perm, size, shape, qs, ks, vs, os, options, scale, dev)
+    return _run_call(q, k, v, out, perm, size, shape, qs, ks, vs, os, options, scale, dev)
+
+
+def _run_call(q, k, v, out, perm, size, shape, qs, ks, vs, os, options, scale, dev):
+    ws = torch.empty(size, dtype=torch.uint8, device=dev)
+    call = _CALL.pack(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 0 if perm is None else perm.data_ptr(),
+                      ws.data_ptr(), size, *shape, *qs[:3], *ks[:3], *vs[:3], *os[:3], *options, scale)
+    _check(lib().vcx_attention_call(call, torch.cuda.current_stream(dev).cuda_stream), "vcx_attention_call")
+    return out
 
 
 FINITE_BLOCKS = 1024  # VCX_FINITE_BLOCKS

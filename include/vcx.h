@@ -222,6 +222,31 @@ int vcx_attention_fwd_fp8(const uint8_t* q8, const uint8_t* k8, const uint8_t* v
                           void* out, int64_t o_sb, int64_t o_sh, int64_t o_sn, uint8_t* p_dump,
                           int64_t p_row_begin, int64_t p_row_end, void* stream);
 
+/* One whole attention call: grouping of V (smooth without perm), preparation of Q, K and V, and
+ * the fused kernel, in the order and with the results of vcx_group_values,
+ * vcx_prepare_qk_int8(_rotated) or vcx_prepare_qk_fp8, vcx_prepare_v_fp8 and
+ * vcx_attention_fwd(_fp8), whose argument rules apply. The payloads live in the caller's
+ * workspace (256-byte aligned, vcx_attention_call_bytes bytes: a function of the shape and the
+ * options, not of the pointers other than whether perm is null), which is free again once the
+ * stream has passed the call. dtype is Q/K/V's and the output's; expcast as for
+ * vcx_attention_fwd; perm (nullable int64 [B,H,Nk]) gathers K and V in place of a grouping;
+ * group_mode, clusters and iterations as for vcx_group_values. Every field is 8 bytes.
+ * Replaces sageattn_vc's chain of native calls
+ * (third_party/sageattention_local/sageattention_local/vc.py:141-197, vc_fp8.py:12-42). */
+typedef struct vcx_call {
+  const void *q, *k, *v;
+  void* out;
+  const int64_t* perm;
+  void* workspace;
+  int64_t workspace_bytes;
+  int64_t B, H, Nq, Nk, D;
+  int64_t q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, v_sb, v_sh, v_sn, o_sb, o_sh, o_sn;
+  int64_t dtype, qk_fp8, rotate, expcast, smooth, channel_scale, clusters, iterations, group_mode;
+  double sm_scale;
+} vcx_call;
+int vcx_attention_call(const vcx_call* call, void* stream);
+int vcx_attention_call_bytes(const vcx_call* call, size_t* bytes);
+
 /* Whether up to three fp16/bf16 arrays (n elements, a multiple of 8, 16-byte aligned; 0 = none)
  * hold a NaN or an infinity: out[0..VCX_FINITE_BLOCKS) (device int32) receives words that are
  * all 0 when every element is finite. Replaces the three torch.isfinite(x).all() of
