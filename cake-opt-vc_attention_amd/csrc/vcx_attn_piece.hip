@@ -18,7 +18,10 @@ __device__ inline void lds_barrier() {
 // every RG-th KB), in the placement of TileLoader. The loads are written as asm: the compiler
 // would drain loads it knows of at every LDS read that might alias them, and here V^T of a
 // tile is in flight while its K is read, and the other way round. Each wave waits for its own
-// loads (wait) before the barrier that hands the region to its readers.
+// loads (wait) before the barrier that hands the region to its readers. The compiler does not
+// place wait states inside asm: s_nop 4 gives the five that an address or resource register
+// needs when a VALU instruction (the read of a spilled scalar, say) has just written it, and the
+// one that M0 needs.
 template <int D, int QF, int RG>
 struct PieceLoader {
   static constexpr int kOps = D / 8;  // 1 KB instructions per operand tile
@@ -52,7 +55,7 @@ struct PieceLoader {
     else rs = rsrc(a.ks + bh * a.tiles * 4, static_cast<uint32_t>(a.tiles * 16));
   }
   __device__ inline static void load16(uint32_t lds, uint32_t voff, const v4i& r, int soff) {
-    asm volatile("s_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+    asm volatile("s_nop 4\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
                  ::"{m0}"(lds), "v"(voff), "s"(r), "s"(soff) : "memory");
   }
   // One of the wave's kPart loads of an operand of tile t into the buffer at byte offset buf.
@@ -65,7 +68,7 @@ struct PieceLoader {
     if (i == 0 && g == 0 && (threadIdx.x & 63) == 0) {
       const uint32_t dst = base + buf + 2 * kTile * D;
       if constexpr (QF == 1)
-        asm volatile("s_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+        asm volatile("s_nop 4\n\tbuffer_load_dword %1, %2, %3 offen lds"
                      ::"{m0}"(dst), "v"(0), "s"(rs), "s"(t * 4) : "memory");
       else load16(dst, 0, rs, t * 16);
     }
