@@ -9,6 +9,8 @@ namespace vcx {
 size_t ws_prepare_qk(int64_t BH, int64_t N, int64_t D);
 size_t ws_prepare_v(int64_t BH, int64_t N, int64_t D);
 size_t ws_group(int64_t BH, int64_t N, int64_t D, int clusters);
+int prepare_together(const vcx_call& c, const int64_t* perm, void* q8, float* qs, void* k8, float* ks, uint8_t* v8,
+                     float* vs, uint16_t* means, void* scratch, void* stream);
 
 namespace {
 
@@ -41,8 +43,8 @@ CallWs call_ws(const vcx_call& c) {
   w.vs = reinterpret_cast<float*>(take(sizeof(float) * BH * c.D * (c.channel_scale ? 1 : tiles)));
   if (c.smooth) w.means = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * BH * tiles * c.D));
   if (groups(c)) w.perm = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * BH * c.Nk));
-  // the stages run one after another on the stream, so they share the scratch
-  w.scratch_bytes = std::max(ws_prepare_qk(BH, c.Nk, c.D), ws_prepare_v(BH, c.Nk, c.D));
+  // grouping and preparation run one after another on the stream, so they share the scratch
+  w.scratch_bytes = ws_prepare_qk(BH, c.Nk, c.D) + ws_prepare_v(BH, c.Nk, c.D);
   if (groups(c)) w.scratch_bytes = std::max(w.scratch_bytes, ws_group(BH, c.Nk, c.D, static_cast<int>(c.clusters)));
   w.scratch = take(w.scratch_bytes);
   w.bytes = off;
@@ -90,22 +92,7 @@ extern "C" int vcx_attention_call(const vcx_call* c, void* stream) {
       return rc;
     perm = w.perm;
   }
-  if (c->qk_fp8) {
-    if (int rc = vcx_prepare_qk_fp8(c->q, c->k, dtype, c->B, c->H, c->Nq, c->Nk, c->D, c->q_sb, c->q_sh, c->q_sn,
-                                    c->k_sb, c->k_sh, c->k_sn, reinterpret_cast<uint8_t*>(w.q8), w.qs,
-                                    reinterpret_cast<uint8_t*>(w.k8), w.ks, nullptr, w.scratch, w.scratch_bytes,
-                                    stream))
-      return rc;
-  } else {
-    auto* prepare = c->rotate ? vcx_prepare_qk_int8_rotated : vcx_prepare_qk_int8;
-    if (int rc = prepare(c->q, c->k, dtype, c->B, c->H, c->Nq, c->Nk, c->D, c->q_sb, c->q_sh, c->q_sn, c->k_sb,
-                         c->k_sh, c->k_sn, perm, w.q8, w.qs, w.k8, w.ks, nullptr, w.scratch, w.scratch_bytes, stream))
-      return rc;
-  }
-  if (int rc = vcx_prepare_v_fp8(c->v, dtype, c->B, c->H, c->Nk, c->D, c->v_sb, c->v_sh, c->v_sn, perm,
-                                 c->smooth != 0, c->channel_scale != 0, w.v8, w.vs, w.means, w.scratch,
-                                 w.scratch_bytes, stream))
-    return rc;
+  if (int rc = prepare_together(*c, perm, w.q8, w.qs, w.k8, w.ks, w.v8, w.vs, w.means, w.scratch, stream)) return rc;
   if (c->qk_fp8)
     return vcx_attention_fwd_fp8(reinterpret_cast<uint8_t*>(w.q8), reinterpret_cast<uint8_t*>(w.k8), w.v8, w.qs, w.ks,
                                  w.vs, c->B, c->H, c->Nq, c->Nk, c->D, static_cast<int>(c->expcast),

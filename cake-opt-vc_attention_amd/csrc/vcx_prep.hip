@@ -16,6 +16,12 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// A [B,H,N,D] tensor: pointer and element strides.
+struct Strided {
+  const void* p;
+  int64_t sb, sh, sn;
+};
+
 template <int D>
 struct Row {
   static constexpr int CPT = D / 16;  // channels per thread
@@ -109,14 +115,15 @@ enum StatsMode { kKSum = 0, kVAmax = 1, kVSmooth = 2 };
 //  kVSmooth: mean[bh][tile][ch] = RN_f32(tile-tree sum / count),
 //            peak[bh][tile][ch] = max |RN(V - mean)| over valid tokens
 template <int DT, int D, int MODE>
-__global__ __launch_bounds__(kThreads) void tile_stats_kernel(
-    const void* x, int64_t H, int64_t n, int64_t sb, int64_t sh, int64_t sn, const int64_t* perm,
-    double* sum_out, float* f_out0, float* f_out1) {
+__device__ __forceinline__ void tile_stats_body(const Strided& t, int64_t H, int64_t n, const int64_t* perm,
+                                                double* sum_out, float* f_out0, float* f_out1, int64_t tile,
+                                                int64_t bh, int64_t tiles) {
+  const void* x = t.p;
+  const int64_t sb = t.sb, sh = t.sh, sn = t.sn;
   constexpr int CPT = D / 16;
   __shared__ double red[4 * D];
   __shared__ float fred[4 * D];
   __shared__ float mean_sh[D];
-  const int64_t tile = blockIdx.x, bh = blockIdx.y, tiles = gridDim.x;
   const int tid = threadIdx.x, kk = tid >> 4, c = tid & 15, lane = tid & 63, w = tid >> 6;
   const uint16_t* base = head_base(x, bh, H, sb, sh);
   // the rows stay packed (16-bit values) and are widened where used: the smoothing
@@ -186,6 +193,22 @@ __global__ __launch_bounds__(kThreads) void tile_stats_kernel(
   }
 }
 
+template <int DT, int D, int MODE>
+__global__ __launch_bounds__(kThreads) void tile_stats_kernel(Strided x, int64_t H, int64_t n, const int64_t* perm,
+                                                              double* sum_out, float* f_out0, float* f_out1) {
+  tile_stats_body<DT, D, MODE>(x, H, n, perm, sum_out, f_out0, f_out1, blockIdx.x, blockIdx.y, gridDim.x);
+}
+
+// The statistics of K (z = 0) and V (z = 1) in one launch: grid (tiles, B*H, 2).
+template <int DT, int D, int VMODE>
+__global__ __launch_bounds__(kThreads) void kv_stats_kernel(Strided k, Strided v, int64_t H, int64_t n,
+                                                            const int64_t* perm, double* ksum, float* v0, float* v1) {
+  if (blockIdx.z == 0)
+    tile_stats_body<DT, D, kKSum>(k, H, n, perm, ksum, nullptr, nullptr, blockIdx.x, blockIdx.y, gridDim.x);
+  else
+    tile_stats_body<DT, D, VMODE>(v, H, n, perm, nullptr, v0, v1, blockIdx.x, blockIdx.y, gridDim.x);
+}
+
 // ---------------------------------------------------------------- finalize
 
 // One thread per channel of head bh. km = RN_in(RN_f32(sum over tiles / n)); also the
@@ -233,12 +256,11 @@ __device__ inline void k_mean_body(const double* sums, int64_t tiles, int64_t n,
 // changes: each thread takes the maximum over its slice of tiles (loads batched), and slice 0
 // combines the slices from LDS.
 constexpr int kScaleThreads = 1024;
-template <bool SMOOTH>
-__global__ __launch_bounds__(kScaleThreads) void v_scale_kernel(const float* a0, const float* a1, int64_t tiles,
-                                                                int D, float* vs, float* recip) {
-  __shared__ float red[2][kScaleThreads];
-  const int64_t bh = blockIdx.x;
-  const int ch = threadIdx.x % D, sl = threadIdx.x / D, S = blockDim.x / D;
+template <bool SMOOTH, int THREADS>
+__device__ __forceinline__ void v_scale_body(const float* a0, const float* a1, int64_t tiles, int D, float* vs,
+                                             float* recip, int64_t bh) {
+  __shared__ float red[2][THREADS];
+  const int ch = threadIdx.x % D, sl = threadIdx.x / D, S = THREADS / D;
   const float* c0 = a0 + bh * tiles * D + ch;
   const float* c1 = SMOOTH ? a1 + bh * tiles * D + ch : nullptr;
   constexpr int kBatch = 8;
@@ -280,16 +302,22 @@ __global__ __launch_bounds__(kScaleThreads) void v_scale_kernel(const float* a0,
   }
 }
 
+template <bool SMOOTH>
+__global__ __launch_bounds__(kScaleThreads) void v_scale_kernel(const float* a0, const float* a1, int64_t tiles,
+                                                                int D, float* vs, float* recip) {
+  v_scale_body<SMOOTH, kScaleThreads>(a0, a1, tiles, D, vs, recip, blockIdx.x);
+}
+
 // ---------------------------------------------------------------- Q INT8
 
 // grid (ceil(n/64), B*H), 256 threads. Groups of rows {16g+t, 16g+t+8}; each
 // group is 32 lanes (16 per row) of one wave; 4 passes of 8 groups.
 // ROT: the rows are rotated by the normalized Hadamard transform (hadamard_row, norm =
 // RN_f32(1/sqrt(D))) in binary32 before the group maximum and the codes.
-// KM (the INT8 Q/K path): blocks (0, bh) instead compute head bh's K mean (k_mean_body, from
-// the K tile sums of the statistics launch before), so that this latency-bound walk runs
-// beside the streaming Q blocks instead of in a launch of its own; the Q blocks are
-// (1 + blk, bh). The K quantization launch that follows reads the mean.
+// quant_q_kernel's blocks (0, bh) instead compute head bh's K mean (k_mean_body, from the K tile
+// sums of the statistics launch before), so that this latency-bound walk runs beside the
+// streaming Q blocks instead of in a launch of its own; the Q blocks are (1 + blk, bh). The K
+// quantization launch that follows reads the mean.
 struct KMeanArgs {
   const double* sums;
   int64_t tiles, n;
@@ -297,20 +325,13 @@ struct KMeanArgs {
   void* km_out;
 };
 
-template <int DT, int D, bool ROT = false, bool KM = false>
-__global__ __launch_bounds__(kThreads) void quant_q_kernel(const void* q, int64_t H, int64_t n,
-                                                           int64_t sb, int64_t sh, int64_t sn,
-                                                           int8_t* q8, float* qs, float norm, KMeanArgs kma) {
+template <int DT, int D, bool ROT>
+__device__ __forceinline__ void quant_q_body(const Strided& q, int64_t H, int64_t n, int8_t* q8, float* qs, float norm,
+                                             int64_t blk, int64_t bh) {
   constexpr int CPT = D / 16;
-  if constexpr (KM) {
-    if (blockIdx.x == 0) {
-      if (threadIdx.x < D) k_mean_body<DT>(kma.sums, kma.tiles, kma.n, D, kma.km, kma.km_out, blockIdx.y, threadIdx.x);
-      return;
-    }
-  }
-  const int64_t blk = KM ? blockIdx.x - 1 : blockIdx.x, bh = blockIdx.y;
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, c = lane & 15, sel = (lane >> 4) & 1;
-  const uint16_t* base = head_base(q, bh, H, sb, sh);
+  const int64_t sn = q.sn;
+  const uint16_t* base = head_base(q.p, bh, H, q.sb, q.sh);
   const int64_t qs_len = (n + 63) / 64 * 32;
   // The four rows of the thread are loaded together before any is used.
   Row<D> rows[4];
@@ -345,6 +366,16 @@ __global__ __launch_bounds__(kThreads) void quant_q_kernel(const void* q, int64_
   }
 }
 
+template <int DT, int D, bool ROT>
+__global__ __launch_bounds__(kThreads) void quant_q_kernel(Strided q, int64_t H, int64_t n, int8_t* q8, float* qs,
+                                                           float norm, KMeanArgs kma) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < D) k_mean_body<DT>(kma.sums, kma.tiles, kma.n, D, kma.km, kma.km_out, blockIdx.y, threadIdx.x);
+    return;
+  }
+  quant_q_body<DT, D, ROT>(q, H, n, q8, qs, norm, blockIdx.x - 1, blockIdx.y);
+}
+
 // ---------------------------------------------------------------- FP8 block Q/K (vc27)
 
 // grid (ceil(n/ROWS), B*H), 256 threads; one block of ROWS rows x D channels shares one
@@ -352,24 +383,16 @@ __global__ __launch_bounds__(kThreads) void quant_q_kernel(const void* q, int64_
 // blk*ROWS + rr + 16*i. x' = CENTER ? RN(x - km) : x (binary32); s = max(RN(amax/448), 1e-12);
 // code = E4M3_satfinite(RN(x'/s)). Rows past n are not part of the block.
 // Reference: quantize_qk_fp8, sal/csrc/vc/qk_fp8.cu:38-74 (Q: 64 rows; K: 128 rows, centred).
-// KM (the Q pass): blocks (0, h) instead compute head h's K mean km = RN_f32(sum / n) from
-// the K statistics (the FP8 path's unrounded mean), so that walk runs beside the Q blocks.
-template <int DT, int D, int ROWS, bool CENTER, bool KM = false>
-__global__ __launch_bounds__(kThreads) void quant_fp8_kernel(const void* x, int64_t H, int64_t n,
-                                                             int64_t sb, int64_t sh, int64_t sn,
-                                                             const float* km, uint8_t* codes, float* scales,
-                                                             KMeanArgs kma) {
-  if constexpr (KM) {
-    if (blockIdx.x == 0) {
-      if (threadIdx.x < D) k_mean_body<DT, true>(kma.sums, kma.tiles, kma.n, D, kma.km, kma.km_out, blockIdx.y, threadIdx.x);
-      return;
-    }
-  }
+// The Q launch's blocks (0, h) instead compute head h's K mean km = RN_f32(sum / n) from the K
+// statistics (the FP8 path's unrounded mean), so that walk runs beside the Q blocks.
+template <int DT, int D, int ROWS, bool CENTER>
+__device__ __forceinline__ void quant_fp8_body(const Strided& x, int64_t H, int64_t n, const float* km, uint8_t* codes,
+                                               float* scales, int64_t blk, int64_t bh, int64_t blocks) {
   constexpr int CPT = D / 16, NR = ROWS / 16;
   __shared__ float wmax[kThreads / 64];
-  const int64_t blk = KM ? blockIdx.x - 1 : blockIdx.x, bh = blockIdx.y, blocks = KM ? gridDim.x - 1 : gridDim.x;
   const int tid = threadIdx.x, rr = tid >> 4, c = tid & 15, lane = tid & 63, w = tid >> 6;
-  const uint16_t* base = head_base(x, bh, H, sb, sh);
+  const int64_t sn = x.sn;
+  const uint16_t* base = head_base(x.p, bh, H, x.sb, x.sh);
   // Every row of the thread is loaded before any is used; Q (read once) non-temporally, so
   // that K stays in the memory-side cache for its own pass.
   Row<D> rows[NR];
@@ -416,6 +439,21 @@ __global__ __launch_bounds__(kThreads) void quant_fp8_kernel(const void* x, int6
     uint8_t* dst = codes + (bh * n + row) * D + c * CPT;
     store_payload_nt<CPT>(dst, packed);
   }
+}
+
+template <int DT, int D>
+__global__ __launch_bounds__(kThreads) void quant_fp8_q_kernel(Strided q, int64_t H, int64_t n, uint8_t* codes,
+                                                               float* scales, KMeanArgs kma) {
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < D) k_mean_body<DT, true>(kma.sums, kma.tiles, kma.n, D, kma.km, kma.km_out, blockIdx.y, threadIdx.x);
+    return;
+  }
+  quant_fp8_body<DT, D, 64, false>(q, H, n, nullptr, codes, scales, blockIdx.x - 1, blockIdx.y, gridDim.x - 1);
+}
+template <int DT, int D>
+__global__ __launch_bounds__(kThreads) void quant_fp8_k_kernel(Strided k, int64_t H, int64_t n, const float* km,
+                                                               uint8_t* codes, float* scales) {
+  quant_fp8_body<DT, D, 128, true>(k, H, n, km, codes, scales, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 // ---------------------------------------------------------------- generic Q/K preprocessing
@@ -572,18 +610,15 @@ __global__ __launch_bounds__(kThreads) void pre_rows_kernel(const void* x, int64
 // grid (tiles, B*H), 256 threads. Thread (kk, c) holds keys kk+16i, all in
 // scale group g = (kk%8)/2; a group is lanes 0-31 or 32-63 of waves w and w+2.
 // ROT: each centred key row k'' is rotated (hadamard_row) in binary32 before quantizing.
-template <int DT, int D, bool ROT = false>
-__global__ __launch_bounds__(kThreads) void quant_k_kernel(const void* k, int64_t H, int64_t n,
-                                                           int64_t sb, int64_t sh, int64_t sn,
-                                                           const int64_t* perm, const float* km,
-                                                           int8_t* k8, float* ks, float norm) {
+template <int DT, int D, bool ROT>
+__device__ __forceinline__ void quant_k_body(const Strided& k, int64_t H, int64_t n, const int64_t* perm,
+                                             const float* km, int8_t* k8, float* ks, float norm, int64_t tile,
+                                             int64_t bh, int64_t tiles) {
   constexpr int CPT = D / 16;
   __shared__ float gred[4][2];
-  // (head, tile) in the reverse order of the statistics pass, so that the rows that pass
-  // read last are still in the memory-side cache when this pass starts.
-  const int64_t tile = gridDim.x - 1 - blockIdx.x, bh = gridDim.y - 1 - blockIdx.y, tiles = gridDim.x;
   const int tid = threadIdx.x, kk = tid >> 4, c = tid & 15, lane = tid & 63, w = tid >> 6;
-  const uint16_t* base = head_base(k, bh, H, sb, sh);
+  const int64_t sn = k.sn;
+  const uint16_t* base = head_base(k.p, bh, H, k.sb, k.sh);
   float mean[CPT];
 #pragma unroll
   for (int j = 0; j < CPT; ++j) mean[j] = km[bh * D + c * CPT + j];
@@ -620,6 +655,15 @@ __global__ __launch_bounds__(kThreads) void quant_k_kernel(const void* k, int64_
   }
 }
 
+// (head, tile) in the reverse order of the statistics pass, so that the rows that pass read
+// last are still in the memory-side cache when this pass starts.
+template <int DT, int D, bool ROT>
+__global__ __launch_bounds__(kThreads) void quant_k_kernel(Strided k, int64_t H, int64_t n, const int64_t* perm,
+                                                           const float* km, int8_t* k8, float* ks, float norm) {
+  quant_k_body<DT, D, ROT>(k, H, n, perm, km, k8, ks, norm, gridDim.x - 1 - blockIdx.x, gridDim.y - 1 - blockIdx.y,
+                           gridDim.x);
+}
+
 // ---------------------------------------------------------------- V E4M3
 
 // grid (tiles, B*H), 256 threads. Bytes are staged in LDS as [D][128] storage
@@ -632,17 +676,16 @@ __global__ __launch_bounds__(kThreads) void quant_k_kernel(const void* k, int64_
 //  SMOOTH = 1: byte = e4m3(RN(RN(x - mean_t) / s)), with s the channel scale
 //              (CHANNEL) or the tile's block scale, written with the fp16 means.
 template <int DT, int D, int SMOOTH, int CHANNEL>
-__global__ __launch_bounds__(kThreads) void quant_v_kernel(
-    const void* vin, int64_t H, int64_t n, int64_t sb, int64_t sh, int64_t sn, const int64_t* perm,
-    const float* scale_or_recip, const float* tile_mean, const float* tile_peak, uint8_t* v8,
-    float* vs_block, uint16_t* means) {
+__device__ __forceinline__ void quant_v_body(const Strided& vin, int64_t H, int64_t n, const int64_t* perm,
+                                             const float* scale_or_recip, const float* tile_mean,
+                                             const float* tile_peak, uint8_t* v8, float* vs_block, uint16_t* means,
+                                             int64_t tile, int64_t bh, int64_t tiles) {
   constexpr int CPG = D / 8;  // channels per thread
   __shared__ __attribute__((aligned(16))) uint8_t stage[D * kTile];
   __shared__ float sc_sh[D], mu_sh[D];
-  // (head, tile) in the reverse order of the statistics pass (see quant_k_kernel).
-  const int64_t tile = gridDim.x - 1 - blockIdx.x, bh = gridDim.y - 1 - blockIdx.y, tiles = gridDim.x;
   const int tid = threadIdx.x, m = tid >> 3, cg = tid & 7;
-  const uint16_t* base = head_base(vin, bh, H, sb, sh);
+  const int64_t sn = vin.sn;
+  const uint16_t* base = head_base(vin.p, bh, H, vin.sb, vin.sh);
   // Row loads first, so that they overlap the scale/mean stage below.
   uint32_t w[4][CPG / 2];
   bool valid[4];
@@ -728,6 +771,75 @@ __global__ __launch_bounds__(kThreads) void quant_v_kernel(
   }
 }
 
+// (head, tile) in the reverse order of the statistics pass (see quant_k_kernel).
+template <int DT, int D, int SMOOTH, int CHANNEL>
+__global__ __launch_bounds__(kThreads) void quant_v_kernel(Strided v, int64_t H, int64_t n, const int64_t* perm,
+                                                           const float* scale_or_recip, const float* tile_mean,
+                                                           const float* tile_peak, uint8_t* v8, float* vs_block,
+                                                           uint16_t* means) {
+  quant_v_body<DT, D, SMOOTH, CHANNEL>(v, H, n, perm, scale_or_recip, tile_mean, tile_peak, v8, vs_block, means,
+                                       gridDim.x - 1 - blockIdx.x, gridDim.y - 1 - blockIdx.y, gridDim.x);
+}
+
+// ---------------------------------------------------------------- Q, K and V together
+
+// The whole preparation in three launches (kv_stats_kernel before these two; prepare_together),
+// where the separate stages take six: the short launches of a small call end to end cost more
+// than their work, and the V scales' walk hides beside the Q blocks. Same box, whole call in us,
+// six launches and three: [1,2,2048,128] 39 / 30, [1,4,1024 x 8192,128] with smoothing 119 / 108,
+// [1,28,8192,128] FP8 541 / 531, [1,7,37741,128] 2472 / 2456, [1,28,37741,128] 9408 / 9395 (there K
+// no longer waits in the memory-side cache between its two passes, and the saved launches
+// make up for it). FMT: 0 INT8, 1 INT8
+// rotated, 2 FP8 blocks. VS: 0 per-channel amax, 1 smoothing with channel scales, 2 with block scales.
+struct PrepOut {
+  void *q8, *k8;
+  uint8_t* v8;
+  float *qs, *ks, *vs;
+  uint16_t* means;
+};
+
+// grid (1 + (VS < 2) + ceil(Nq/64), B*H): the K mean, the V scales, then the Q blocks.
+template <int DT, int D, int FMT, int VS>
+__global__ __launch_bounds__(kThreads) void prep_q_kernel(Strided q, int64_t H, int64_t n, PrepOut o, float norm,
+                                                          KMeanArgs kma, const float* a0, const float* a1,
+                                                          float* recip) {
+  constexpr int kFirst = VS == 2 ? 1 : 2;
+  const int64_t bh = blockIdx.y;
+  if (blockIdx.x == 0) {
+    if (threadIdx.x < D) k_mean_body<DT, FMT == 2>(kma.sums, kma.tiles, kma.n, D, kma.km, kma.km_out, bh, threadIdx.x);
+    return;
+  }
+  if constexpr (VS < 2) {
+    if (blockIdx.x == 1) {
+      v_scale_body<VS == 1, kThreads>(a0, a1, kma.tiles, D, o.vs, recip, bh);
+      return;
+    }
+  }
+  const int64_t blk = static_cast<int64_t>(blockIdx.x) - kFirst;
+  if constexpr (FMT == 2)
+    quant_fp8_body<DT, D, 64, false>(q, H, n, nullptr, static_cast<uint8_t*>(o.q8), o.qs, blk, bh, gridDim.x - kFirst);
+  else
+    quant_q_body<DT, D, FMT == 1>(q, H, n, static_cast<int8_t*>(o.q8), o.qs, norm, blk, bh);
+}
+
+// grid (tiles, B*H, 2): K (z = 0) and V (z = 1).
+template <int DT, int D, int FMT, int VS>
+__global__ __launch_bounds__(kThreads) void prep_kv_kernel(Strided k, Strided v, int64_t H, int64_t n,
+                                                           const int64_t* perm, PrepOut o, float norm,
+                                                           const float* km, const float* a0, const float* a1,
+                                                           const float* recip) {
+  const int64_t tile = blockIdx.x, bh = blockIdx.y, tiles = gridDim.x;
+  if (blockIdx.z == 0) {
+    if constexpr (FMT == 2)
+      quant_fp8_body<DT, D, 128, true>(k, H, n, km, static_cast<uint8_t*>(o.k8), o.ks, tile, bh, tiles);
+    else
+      quant_k_body<DT, D, FMT == 1>(k, H, n, perm, km, static_cast<int8_t*>(o.k8), o.ks, norm, tile, bh, tiles);
+  } else {
+    quant_v_body<DT, D, VS != 0, VS != 2>(v, H, n, perm, VS == 0 ? recip : o.vs, a0, a1, o.v8, o.vs, o.means, tile, bh,
+                                          tiles);
+  }
+}
+
 // ---------------------------------------------------------------- probes
 
 __global__ void expcast_kernel(const float* x, uint8_t* y, int64_t n) {
@@ -780,11 +892,6 @@ __global__ __launch_bounds__(256) void finite_kernel(FiniteArgs a, uint32_t mask
 }
 
 // ---------------------------------------------------------------- host helpers
-
-struct Strided {
-  const void* p;
-  int64_t sb, sh, sn;
-};
 
 int check_input(const char* name, const void* p, int64_t B, int64_t H, int64_t N, int64_t D,
                 int64_t sb, int64_t sh, int64_t sn) {
@@ -862,25 +969,20 @@ int prepare_qk_int8(const void* q, const void* k, int dtype, int64_t B, int64_t 
   // K statistics, then the Q quantization with the K mean in its first blocks, then the K
   // quantization.
   const KMeanArgs kma{ksum, tiles, Nk, km, km_out};
+  const Strided qt{q, q_sb, q_sh, q_sn}, kt{k, k_sb, k_sh, k_sn};
   return dispatch(dtype, D, [&](auto dt, auto dd) -> int {
     constexpr int DT = decltype(dt)::value, DD = decltype(dd)::value;
-    tile_stats_kernel<DT, DD, kKSum><<<dim3(tiles, BH), kThreads, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, perm,
-                                                                          ksum, nullptr, nullptr);
+    tile_stats_kernel<DT, DD, kKSum><<<dim3(tiles, BH), kThreads, 0, st>>>(kt, H, Nk, perm, ksum, nullptr, nullptr);
     VCX_LAUNCHED("tile_stats_kernel<K>");
-    const dim3 qgrid(cdiv(Nq, 64) + 1, BH);
-    if (rotate)
-      quant_q_kernel<DT, DD, true, true><<<qgrid, kThreads, 0, st>>>(q, H, Nq, q_sb, q_sh, q_sn, q8, qs, norm, kma);
-    else
-      quant_q_kernel<DT, DD, false, true><<<qgrid, kThreads, 0, st>>>(q, H, Nq, q_sb, q_sh, q_sn, q8, qs, norm, kma);
-    VCX_LAUNCHED("quant_q_kernel");
-    if (rotate)
-      quant_k_kernel<DT, DD, true><<<dim3(tiles, BH), kThreads, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, perm, km, k8,
-                                                                        ks, norm);
-    else
-      quant_k_kernel<DT, DD><<<dim3(tiles, BH), kThreads, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, perm, km, k8, ks,
-                                                                  norm);
-    VCX_LAUNCHED("quant_k_kernel");
-    return VCX_OK;
+    auto quant = [&](auto rot) -> int {
+      constexpr bool ROT = decltype(rot)::value;
+      quant_q_kernel<DT, DD, ROT><<<dim3(cdiv(Nq, 64) + 1, BH), kThreads, 0, st>>>(qt, H, Nq, q8, qs, norm, kma);
+      VCX_LAUNCHED("quant_q_kernel");
+      quant_k_kernel<DT, DD, ROT><<<dim3(tiles, BH), kThreads, 0, st>>>(kt, H, Nk, perm, km, k8, ks, norm);
+      VCX_LAUNCHED("quant_k_kernel");
+      return VCX_OK;
+    };
+    return rotate ? quant(std::true_type()) : quant(std::false_type());
   });
 }
 }  // namespace
@@ -904,6 +1006,58 @@ extern "C" int vcx_prepare_qk_int8_rotated(const void* q, const void* k, int dty
   return prepare_qk_int8(q, k, dtype, B, H, Nq, Nk, D, q_sb, q_sh, q_sn, k_sb, k_sh, k_sn, perm, q8, qs, k8, ks,
                          km_out, workspace, workspace_bytes, stream, true);
 }
+
+// Q, K and V of one call in three launches. Outputs and results are those of
+// vcx_prepare_qk_int8(_rotated) or vcx_prepare_qk_fp8, and vcx_prepare_v_fp8. The scratch holds
+// both stages' workspaces.
+namespace vcx {
+int prepare_together(const vcx_call& c, const int64_t* perm, void* q8, float* qs, void* k8, float* ks, uint8_t* v8,
+                     float* vs, uint16_t* means, void* scratch, void* stream) {
+  if (int rc = check_shape(c.B, c.H, c.Nq, c.D)) return rc;
+  if (int rc = check_shape(c.B, c.H, c.Nk, c.D)) return rc;
+  VCX_REQUIRE(c.dtype == VCX_FLOAT16 || c.dtype == VCX_BFLOAT16, "dtype must be float16 or bfloat16");
+  if (int rc = check_input("q", c.q, c.B, c.H, c.Nq, c.D, c.q_sb, c.q_sh, c.q_sn)) return rc;
+  if (int rc = check_input("k", c.k, c.B, c.H, c.Nk, c.D, c.k_sb, c.k_sh, c.k_sn)) return rc;
+  if (int rc = check_input("v", c.v, c.B, c.H, c.Nk, c.D, c.v_sb, c.v_sh, c.v_sn)) return rc;
+  VCX_REQUIRE(aligned(perm, 8), "perm misaligned");
+  const int64_t BH = c.B * c.H, tiles = cdiv(c.Nk, kTile);
+  auto* ws = static_cast<char*>(scratch);
+  double* ksum = reinterpret_cast<double*>(ws);
+  float* km = reinterpret_cast<float*>(ws + align_up(sizeof(double) * BH * tiles * c.D));
+  ws += ws_prepare_qk(BH, c.Nk, c.D);
+  const size_t slice = align_up(sizeof(float) * BH * tiles * c.D);
+  float* a0 = reinterpret_cast<float*>(ws);
+  float* a1 = reinterpret_cast<float*>(ws + slice);
+  float* recip = reinterpret_cast<float*>(ws + 2 * slice);
+  const KMeanArgs kma{ksum, tiles, c.Nk, km, nullptr};
+  const Strided q{c.q, c.q_sb, c.q_sh, c.q_sn}, k{c.k, c.k_sb, c.k_sh, c.k_sn}, v{c.v, c.v_sb, c.v_sh, c.v_sn};
+  const PrepOut o{q8, k8, v8, qs, ks, vs, means};
+  const float norm = static_cast<float>(1.0 / std::sqrt(static_cast<double>(c.D)));
+  hipStream_t st = static_cast<hipStream_t>(stream);
+  return dispatch(static_cast<int>(c.dtype), c.D, [&](auto dt, auto dd) -> int {
+    constexpr int DT = decltype(dt)::value, DD = decltype(dd)::value;
+    auto run = [&](auto fmt, auto value) -> int {
+      constexpr int FMT = decltype(fmt)::value, VS = decltype(value)::value;
+      const dim3 both(static_cast<unsigned>(tiles), static_cast<unsigned>(BH), 2);
+      kv_stats_kernel<DT, DD, VS == 0 ? kVAmax : kVSmooth><<<both, kThreads, 0, st>>>(k, v, c.H, c.Nk, perm, ksum, a0, a1);
+      VCX_LAUNCHED("kv_stats_kernel");
+      prep_q_kernel<DT, DD, FMT, VS><<<dim3(static_cast<unsigned>(cdiv(c.Nq, 64) + (VS == 2 ? 1 : 2)),
+                                            static_cast<unsigned>(BH)), kThreads, 0, st>>>(q, c.H, c.Nq, o, norm, kma,
+                                                                                           a0, a1, recip);
+      VCX_LAUNCHED("prep_q_kernel");
+      prep_kv_kernel<DT, DD, FMT, VS><<<both, kThreads, 0, st>>>(k, v, c.H, c.Nk, perm, o, norm, km, a0, a1, recip);
+      VCX_LAUNCHED("prep_kv_kernel");
+      return VCX_OK;
+    };
+    auto format = [&](auto fmt) -> int {
+      if (!c.smooth) return run(fmt, std::integral_constant<int, 0>());
+      return c.channel_scale ? run(fmt, std::integral_constant<int, 1>()) : run(fmt, std::integral_constant<int, 2>());
+    };
+    if (c.qk_fp8) return run(std::integral_constant<int, 2>(), std::integral_constant<int, 0>());
+    return c.rotate ? format(std::integral_constant<int, 1>()) : format(std::integral_constant<int, 0>());
+  });
+}
+}  // namespace vcx
 
 // ---------------------------------------------------------------- allocation-free variant
 
@@ -981,16 +1135,14 @@ extern "C" int vcx_prepare_qk_fp8(const void* q, const void* k, int dtype, int64
     constexpr int DT = decltype(dt)::value, DD = decltype(dd)::value;
     // K statistics, then the Q quantization with the K mean in its first blocks (Q read
     // non-temporally, so K stays in the memory-side cache), then the K quantization.
-    tile_stats_kernel<DT, DD, kKSum><<<dim3(tiles, BH), kThreads, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, nullptr,
-                                                                          ksum, nullptr, nullptr);
+    const Strided qt{q, q_sb, q_sh, q_sn}, kt{k, k_sb, k_sh, k_sn};
+    tile_stats_kernel<DT, DD, kKSum><<<dim3(tiles, BH), kThreads, 0, st>>>(kt, H, Nk, nullptr, ksum, nullptr, nullptr);
     VCX_LAUNCHED("tile_stats_kernel<K>");
     const KMeanArgs kma{ksum, tiles, Nk, km, km_out};
-    quant_fp8_kernel<DT, DD, 64, false, true><<<dim3(cdiv(Nq, 64) + 1, BH), kThreads, 0, st>>>(
-        q, H, Nq, q_sb, q_sh, q_sn, nullptr, q8, qs, kma);
-    VCX_LAUNCHED("quant_fp8_kernel<Q>");
-    quant_fp8_kernel<DT, DD, 128, true><<<dim3(tiles, BH), kThreads, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, km, k8,
-                                                                              ks, KMeanArgs{});
-    VCX_LAUNCHED("quant_fp8_kernel<K>");
+    quant_fp8_q_kernel<DT, DD><<<dim3(cdiv(Nq, 64) + 1, BH), kThreads, 0, st>>>(qt, H, Nq, q8, qs, kma);
+    VCX_LAUNCHED("quant_fp8_q_kernel");
+    quant_fp8_k_kernel<DT, DD><<<dim3(tiles, BH), kThreads, 0, st>>>(kt, H, Nk, km, k8, ks);
+    VCX_LAUNCHED("quant_fp8_k_kernel");
     return VCX_OK;
   });
 }
@@ -1019,27 +1171,26 @@ extern "C" int vcx_prepare_v_fp8(const void* v, int dtype, int64_t B, int64_t H,
   hipStream_t st = static_cast<hipStream_t>(stream);
   return dispatch(dtype, D, [&](auto dt, auto dd) -> int {
     constexpr int DT = decltype(dt)::value, DD = decltype(dd)::value;
-    dim3 grid(tiles, BH);
+    const dim3 grid(tiles, BH);
+    const Strided vt{v, v_sb, v_sh, v_sn};
     if (!smooth) {
-      tile_stats_kernel<DT, DD, kVAmax><<<grid, kThreads, 0, st>>>(v, H, N, v_sb, v_sh, v_sn, perm, nullptr, a0, nullptr);
+      tile_stats_kernel<DT, DD, kVAmax><<<grid, kThreads, 0, st>>>(vt, H, N, perm, nullptr, a0, nullptr);
       VCX_LAUNCHED("tile_stats_kernel<Vamax>");
       v_scale_kernel<false><<<dim3(BH), kScaleThreads / DD * DD, 0, st>>>(a0, nullptr, tiles, DD, vs, recip);
       VCX_LAUNCHED("v_scale_kernel");
-      quant_v_kernel<DT, DD, 0, 1><<<grid, kThreads, 0, st>>>(v, H, N, v_sb, v_sh, v_sn, perm, recip, nullptr,
-                                                              nullptr, v8, nullptr, nullptr);
+      quant_v_kernel<DT, DD, 0, 1><<<grid, kThreads, 0, st>>>(vt, H, N, perm, recip, nullptr, nullptr, v8, nullptr,
+                                                              nullptr);
       VCX_LAUNCHED("quant_v_kernel");
       return VCX_OK;
     }
-    tile_stats_kernel<DT, DD, kVSmooth><<<grid, kThreads, 0, st>>>(v, H, N, v_sb, v_sh, v_sn, perm, nullptr, a0, a1);
+    tile_stats_kernel<DT, DD, kVSmooth><<<grid, kThreads, 0, st>>>(vt, H, N, perm, nullptr, a0, a1);
     VCX_LAUNCHED("tile_stats_kernel<Vsmooth>");
     if (channel_scale) {
       v_scale_kernel<true><<<dim3(BH), kScaleThreads / DD * DD, 0, st>>>(a0, a1, tiles, DD, vs, nullptr);
       VCX_LAUNCHED("v_scale_kernel");
-      quant_v_kernel<DT, DD, 1, 1><<<grid, kThreads, 0, st>>>(v, H, N, v_sb, v_sh, v_sn, perm, vs, a0, a1, v8,
-                                                              nullptr, means);
+      quant_v_kernel<DT, DD, 1, 1><<<grid, kThreads, 0, st>>>(vt, H, N, perm, vs, a0, a1, v8, nullptr, means);
     } else {
-      quant_v_kernel<DT, DD, 1, 0><<<grid, kThreads, 0, st>>>(v, H, N, v_sb, v_sh, v_sn, perm, nullptr, a0, a1,
-                                                              v8, vs, means);
+      quant_v_kernel<DT, DD, 1, 0><<<grid, kThreads, 0, st>>>(vt, H, N, perm, nullptr, a0, a1, v8, vs, means);
     }
     VCX_LAUNCHED("quant_v_kernel");
     return VCX_OK;
