@@ -291,6 +291,27 @@ __device__ __forceinline__ void attn_piece(const AttnArgs& a, int64_t bh, int64_
 template <int RG>
 constexpr int kSplits = 8 / RG;
 constexpr int kPieceThreads = 512;
+constexpr int kWarm = 4;  // loads per thread of warm_l2
+
+// One 128-byte line per load of the head's first tiles, shared out over the n pieces of the head
+// on this XCD (this is the i-th): the pieces walk the tiles together, so without it every step
+// waits for its tile from memory; with it for the XCD's L2. Nothing waits for these loads but
+// the first tile's wait, which runs beside them. In calls that have just written K and V: [1,4,1024
+// x 8192,128] with smoothing 51.9 -> 39.2 us, [1,2,2048,128] 15.0 -> 13.9 us.
+template <int D>
+__device__ __forceinline__ void warm_l2(const AttnArgs& a, int64_t bh, int64_t i, int64_t n, uint32_t (&sink)[kWarm]) {
+  const int64_t npad = a.tiles * kTile, lines = a.tiles * 2 * D, valid = a.Nk * D / 128;
+  const uint8_t* k = reinterpret_cast<const uint8_t*>(a.k8) + bh * a.Nk * D;
+  const uint8_t* v = a.v8 + bh * D * npad;
+#pragma unroll
+  for (int e = 0; e < kWarm; ++e) {
+    // lines in the order of the tiles: D of K, then D of V^T (one per channel)
+    const int64_t l = (e * n + i) * kPieceThreads + threadIdx.x, t = l / (2 * D), r = l % (2 * D);
+    const int64_t kl = t * D + r;
+    const uint8_t* p = r < D ? k + (kl < valid ? kl : 0) * 128 : v + (r - D) * npad + t * kTile;
+    sink[e] = *reinterpret_cast<const uint32_t*>(l < lines ? p : v);
+  }
+}
 
 template <int D, int VM, int PM, int QF, int RG>
 __global__ __launch_bounds__(kPieceThreads, 1) void attn_piece_kernel(AttnArgs a) {
@@ -302,8 +323,15 @@ __global__ __launch_bounds__(kPieceThreads, 1) void attn_piece_kernel(AttnArgs a
   // contiguous (head, row) ranges per XCD, as in attn_kernel
   const int64_t per = gridDim.x / 8, rem = gridDim.x % 8, xcd = blockIdx.x % 8, j = blockIdx.x / 8;
   const int64_t logical = (xcd < rem ? xcd * (per + 1) : rem * (per + 1) + (xcd - rem) * per) + j;
-  const int64_t pieces = (a.Nq + kRows - 1) / kRows;
-  attn_piece<D, VM, PM, QF, RG, KS, DB>(a, logical / pieces, logical % pieces * kRows, lds, xch);
+  const int64_t pieces = (a.Nq + kRows - 1) / kRows, bh = logical / pieces;
+  // this XCD's pieces of the head
+  const int64_t lo0 = logical - j, hi0 = lo0 + per + (xcd < rem ? 1 : 0);
+  const int64_t lo = lo0 > bh * pieces ? lo0 : bh * pieces, hi = hi0 < (bh + 1) * pieces ? hi0 : (bh + 1) * pieces;
+  uint32_t sink[kWarm];
+  warm_l2<D>(a, bh, logical - lo, hi - lo, sink);
+  attn_piece<D, VM, PM, QF, RG, KS, DB>(a, bh, logical % pieces * kRows, lds, xch);
+#pragma unroll
+  for (int e = 0; e < kWarm; ++e) asm volatile("" ::"v"(sink[e]));  // the loads are used
 #else
   (void)a;
 #endif
