@@ -331,6 +331,21 @@ def test_grouping_many_clusters_bit_exact(dim, n, clusters, iterations):
     np.testing.assert_array_equal(perm.cpu().numpy(), eperm)
 
 
+@pytest.mark.parametrize("n,clusters", [(1, 8), (128, 5), (129, 8), (1024 * 128, 8), (1024 * 128 + 1, 3)])
+def test_grouping_sort_of_few_labels(n, clusters):
+    # Up to 8 labels and 1024 tiles are sorted by one launch whose blocks sum the head's counts
+    # (128 tiles per pass); past that by two launches. Two heads; two clusters without a token
+    # among eight where the values leave them. The permutation is the stable sort of the labels.
+    _print_case("grouping sort", n, clusters)
+    g = torch.Generator().manual_seed(n)
+    v = torch.randn(1, 2, n, 64, generator=g) * 0.1
+    v[..., 0] += torch.randint(0, 6, (1, 2, n), generator=g) * 3.0
+    v = v.to(torch.bfloat16).to(DEV)
+    perm, labels, _ = vcx.group_values(v, clusters, 2, debug=True)
+    assert int(labels.max()) < min(clusters, n)
+    assert torch.equal(perm, labels.sort(dim=-1, stable=True).indices)
+
+
 @pytest.mark.parametrize("dim,dtype", [(64, torch.float16), (128, torch.bfloat16)])
 @pytest.mark.parametrize("n,clusters", [(256 * 128, 9), (256 * 128 + 1, 9), (512 * 128 - 1, 200)])
 def test_grouping_sorted_update_at_its_tile_chunks(dim, dtype, n, clusters):
