@@ -45,7 +45,7 @@
 // attn_utils.cuh:355-455): a.sm = RN(sm * RN(log2 e)), base/factor as above,
 // m' = max(m, max fmaf(base, factor, -8.807)), P = E4M3(exp2(fmaf(base, factor, -m'))) with
 // the correctly rounded binary32 exp2 (fp8_exp2_word: v_exp_f32, rechecked in binary64 next
-// to an E4M3 rounding midpoint); den and the mean restore use the unrounded sum of P.
+// to an E4M3 rounding midpoint, which fp8_exp2_gap looks for); den and the mean restore use the unrounded sum of P.
 #include "vcx_attn.hpp"
 
 #include <functional>
@@ -71,7 +71,9 @@ __device__ __forceinline__ void body_tiles(W& w, const LD& ld, const AttnArgs& a
                                            uint8_t* lds1, uint8_t* meta0, uint8_t* meta1) {
   constexpr int KB = kTile * W::kD;
   const TI body = static_cast<TI>(a.tiles) - 1;
-  for (; t + 2 <= body; t += 2) {
+  constexpr bool kLeaves = PRE && W::kPM == 0;  // a wave may leave this copy for the other one
+  TI end = body;
+  for (; t + 2 <= end; t += 2) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     w.template tile<false, PRE>(a, t, lds0, lds0 + KB, meta0, [&](int i) {
@@ -82,8 +84,9 @@ __device__ __forceinline__ void body_tiles(W& w, const LD& ld, const AttnArgs& a
     w.template tile<false, PRE>(a, t + 1, lds1, lds1 + KB, meta1, [&](int i) {
       if (i < LD::kParts) ld.part(i, t + 2, lds0, lds0 + KB, meta0);
     });
+    if constexpr (kLeaves) end = wave_any(w.wide != 0) ? 0 : body;
   }
-  if (t < body) {  // odd count of body tiles: one more from buffer 0, last tile lands in buffer 1
+  if (kLeaves ? t + 1 == body : t < body) {  // odd count of body tiles: one more from buffer 0, last tile lands in buffer 1
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     w.template tile<false, PRE>(a, t, lds0, lds0 + KB, meta0, [&](int i) {
@@ -169,7 +172,12 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, int64_t bh, int64_
   // per-block-scale variants keep 64 bits (with 32 their register allocation spills)
   typedef std::conditional_t<VM == 2, int64_t, int> TI;
   TI t = 0;
-  if constexpr (PM == 2 && QF == 0) {
+  w.wide = 0;
+  if constexpr (PM == 0) {
+    // the cheap midpoint test until a vanishing probability; after an early end the rest
+    body_tiles<true>(w, ld, a, t, lds0, lds1, meta0, meta1);
+    body_tiles<false>(w, ld, a, t, lds0, lds1, meta0, meta1);
+  } else if constexpr (PM == 2 && QF == 0) {
     if (w.fold_ok) body_tiles<true>(w, ld, a, t, lds0, lds1, meta0, meta1);
     else body_tiles<false>(w, ld, a, t, lds0, lds1, meta0, meta1);
   } else {

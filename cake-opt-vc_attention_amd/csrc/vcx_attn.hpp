@@ -264,7 +264,7 @@ struct Wave {
   // scales keep v_cvt_f32_i32: the bias register costs them spills.
   static constexpr bool IB = QF == 0 && (PM == 2 || (PM == 1 && D == 128 && VM == 1) ||
                                          (PM == 0 && D == 128 && !(VM == 2 && DUMP)));
-  static constexpr int kD = D;
+  static constexpr int kD = D, kPM = PM;
   static constexpr int DS = D / 64;  // 64-deep QK steps
   static constexpr int CB = D / 16;  // 16-channel output blocks
   static constexpr bool SMOOTH = VM >= 1, BSCALE = VM == 2;
@@ -297,6 +297,7 @@ struct Wave {
   // Folded encode (INT8 QK): the per-tile fold conditions are known to hold on every tile
   // but the last (set once per wave by fold_precheck; wave-uniform)
   int fold_ok;
+  int wide;  // control path: the wave has met a vanishing probability
   int G, li;
   int64_t bh_;
 
@@ -508,7 +509,7 @@ struct Wave {
   // the control path the row's unrounded mass tmq).
   template <bool LAST, bool PRE>
   __device__ __forceinline__ void bytes(const AttnArgs& a, const float (&bs)[8][4], float scl, float mx, float fb,
-                                        v8i& Pq, float& tmq) const {
+                                        v8i& Pq, float& tmq) {
     if constexpr (PM == 2) {
       // Folded ExpCast encode (the reference's default kernel modes without block
       // values, sal/csrc/vc/vc_math.cuh:16-111): code = RNE(fmaf(base, gain, bias)) with
@@ -559,34 +560,44 @@ struct Wave {
         Pq[j] = static_cast<int>(w);
       }
     } else {
+      // E4M3 of the hardware exp2, unless a probability of the span (a tile, at D64 four: its
+      // three waves per SIMD have no registers for more) may lie within two ulps of an E4M3
+      // midpoint by fp8_exp2_gap (a few in a hundred thousand): then the lane redoes the span
+      // from the scores, which stay live, with both neighbours' bytes, and in binary64 where
+      // these differ. One branch per tile keeps the loop one block that the MFMAs interleave with.
+      // A vanishing probability (a score more than about 103 nats below the row maximum) always
+      // fails the test: PRE takes none into account but sets wide, upon which the wave leaves for
+      // the copy of the loop that lifts small probabilities over it, one more instruction per
+      // probability. Same box, us, both neighbours' bytes of every probability / lifted / this:
+      // smoothing [1,7,37741,128] 3830 / 3703 / 3528, [1,8,16000,64] 696 / 638 / 601, [1,16,3000,128]
+      // 94.4 / 92.1 / 87.3. With Q scaled by 25, where every wave leaves after its first two
+      // tiles: 3674 / 3460 / 3513, 689 / 627 / 648, 88.6 / 85.5 / 91.7.
       const float f = scl;
-      // Bytes of the +-2 ulp neighbours of every probability (the lower ones by a saturating
-      // subtraction on every tile, so that p = 0, i.e. a score more than about 103 nats
-      // below the row maximum, never forces a recheck); an E4M3 midpoint within two ulps
-      // (the neighbours disagree, a few lanes per million) takes the binary64 recheck.
-      // At D128 the recheck is one branch per tile (a lane that missed redoes its tile from
-      // the scores, which stay live), so the loop stays one block that the MFMAs
-      // interleave with; D64's three waves per SIMD have no registers for that and branch
-      // per four probabilities.
       float ls = -0.0f;  // -0 + p = p: the first addition folds away
-      if constexpr (D == 128) {
-        uint32_t miss = 0;
+      constexpr int kSpan = D == 128 ? 8 : 1;
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+      for (int j0 = 0; j0 < 8; j0 += kSpan) {
+        const float ls0 = ls;
+        uint32_t gap = 0xffffffffu;
+#pragma unroll
+        for (int j = j0; j < j0 + kSpan; ++j) {
           float pr[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) pr[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(bs[j][r], f, -mx));
-          uint32_t lo, hi;
-          fp8_exp2_bounds<true, true>(pr, lo, hi);
-          Pq[j] = static_cast<int>(lo);
-          miss |= lo ^ hi;
 #pragma unroll
-          for (int r = 0; r < 4; ++r) ls += pr[r];
+          for (int r = 0; r < 4; ++r) {
+            const uint32_t g = fp8_exp2_gap<!PRE>(pr[r]);
+            gap = gap < g ? gap : g;
+            ls += pr[r];
+          }
+          const int w = __builtin_amdgcn_cvt_pk_fp8_f32(pr[0], pr[1], 0, false);
+          Pq[j] = __builtin_amdgcn_cvt_pk_fp8_f32(pr[2], pr[3], w, true);
         }
-        if (__builtin_expect(miss != 0, 0)) {
-          ls = -0.0f;
+        if (__builtin_expect(gap <= kFp8Gap, 0)) {
+          ls = ls0;
+          float low = 1.0f;
 #pragma unroll
-          for (int j = 0; j < 8; ++j) {
+          for (int j = j0; j < j0 + kSpan; ++j) {
             float xs[4], pr[4];
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
@@ -594,24 +605,13 @@ struct Wave {
               asm volatile("" : "+v"(b));  // recomputed here, not kept live from the loop above
               xs[r] = __builtin_fmaf(b, f, -mx);
               pr[r] = __builtin_amdgcn_exp2f(xs[r]);
+              low = fminf(low, pr[r]);
             }
             Pq[j] = static_cast<int>(fp8_exp2_word<true>(xs, pr));
 #pragma unroll
             for (int r = 0; r < 4; ++r) ls += pr[r];
           }
-        }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          float xs[4], pr[4];
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            xs[r] = __builtin_fmaf(bs[j][r], f, -mx);
-            pr[r] = __builtin_amdgcn_exp2f(xs[r]);
-          }
-          Pq[j] = static_cast<int>(fp8_exp2_word<true>(xs, pr));
-#pragma unroll
-          for (int r = 0; r < 4; ++r) ls += pr[r];
+          if constexpr (PRE) wide |= low < 0x1p-100f ? 1 : 0;
         }
       }
       tmq = row_sum(ls);

@@ -108,13 +108,12 @@ __device__ inline uint32_t e4m3_sat(float x) {
 // input). The bytes of p - 2 ulps and p + 2 ulps agree unless an E4M3 rounding midpoint lies
 // within two ulps of p; only then does the lane recompute exp2 in binary64 and round it once
 // to binary32 (p is updated to that value). The upper neighbours of two probabilities come
-// from one 64-bit add (v_lshl_add_u64). SAT = true (what the fused kernel uses) forms the
+// from one 64-bit add (v_lshl_add_u64). SAT = true (what the fused kernel's recheck uses) forms the
 // lower neighbours with a saturating subtraction per probability. SAT = false uses one 64-bit
 // subtraction per pair, half the instructions, but a borrow out of a low half below 2 ulps (p
 // = 0 or the smallest subnormal, i.e. x below about -149) then yields a NaN byte and a
 // needless recheck: bytes stay right, but rows whose scores lie more than about 103 nats
-// below the row maximum recheck on most tiles. Same-box A/B of the control path: SAT costs
-// 5.8 % (D128) and 11 % (D64) on N(0,1) scores and is 4-5 times faster with Q scaled by 25.
+// below the row maximum recheck on most tiles. The fused kernel asks fp8_exp2_gap first.
 // Reference: the probability byte of sal/sageattention_local/vc_reference.py:68-75 and
 // sal/csrc/qattn/attn_utils.cuh:355-455.
 // fp8_exp2_bounds gives the bytes of both neighbour sets (lo, hi); fp8_exp2_word resolves a
@@ -122,7 +121,7 @@ __device__ inline uint32_t e4m3_sat(float x) {
 // recheck.
 __device__ __noinline__ inline float exp2_via_f64(float x) { return static_cast<float>(exp2(static_cast<double>(x))); }
 
-template <bool SAT = false, bool REUSE = false>
+template <bool SAT>
 __device__ inline void fp8_exp2_bounds(const float (&p)[4], uint32_t& lo, uint32_t& hi) {
   constexpr uint64_t kTwoUlps = 0x0000000200000002ull;
   float dn[4], up[4];
@@ -142,12 +141,9 @@ __device__ inline void fp8_exp2_bounds(const float (&p)[4], uint32_t& lo, uint32
       dn[2 * h + 1] = __uint_as_float(static_cast<uint32_t>(d >> 32));
     }
   }
-  // REUSE: the first conversion of each word writes its low half over an input that dies
-  // there (the high half is written next) instead of a zeroed register; one move less per
-  // word, at the price of a longer-lived input where registers are short
-  lo = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(dn[0], dn[1], REUSE ? __float_as_int(dn[0]) : 0, false));
+  lo = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(dn[0], dn[1], 0, false));
   lo = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(dn[2], dn[3], static_cast<int>(lo), true));
-  hi = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(up[0], up[1], REUSE ? __float_as_int(up[0]) : 0, false));
+  hi = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(up[0], up[1], 0, false));
   hi = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(up[2], up[3], static_cast<int>(hi), true));
 }
 
@@ -164,6 +160,21 @@ __device__ inline uint32_t fp8_exp2_word(const float (&x)[4], float (&p)[4]) {
     lo = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(p[2], p[3], static_cast<int>(lo), true));
   }
   return lo;
+}
+
+// A cheaper first test: every E4M3 rounding midpoint has at most four bits after the leading
+// one, i.e. its low 19 bits are zero in binary32 (normal results four, subnormal ones and the
+// edge to zero at most three), so no midpoint lies within two ulps of p unless
+// fp8_exp2_gap(p) <= kFp8Gap; else p's own byte is the byte. It also holds next to the E4M3
+// values themselves and at p = 0. LIFT: p below 2^-64, far below the smallest midpoint 2^-10,
+// is taken as a value that passes (as integers, so that a NaN still fails).
+constexpr uint32_t kFp8Gap = 4u << 13;
+template <bool LIFT>
+__device__ inline uint32_t fp8_exp2_gap(float p) {
+  constexpr uint32_t kLift = (127u - 64u) << 23 | 1u << 18;
+  uint32_t u = __float_as_uint(p);
+  if constexpr (LIFT) u = u > kLift ? u : kLift;
+  return (u << 13) + (2u << 13);
 }
 
 // ExpCast constants (exact fp32 values of the reference, expcast.cuh:7).

@@ -801,6 +801,32 @@ def test_control_path_far_logits_p_bytes_and_output(dim):
     assert cosine(got, eout) >= 0.9999
 
 
+@pytest.mark.parametrize("dim,nk", [(64, 130), (64, 640), (64, 700), (128, 256), (128, 513), (128, 768)])
+def test_control_path_vanishing_probabilities_from_some_tile_on(dim, nk):
+    # 257 heads, so that the call takes the 128-row blocks: head h meets scores more than 103
+    # nats below the row maximum first in tile h % (tiles + 1) (the last class: nowhere), so its
+    # waves leave the loop of the cheap midpoint test after every pair of tiles, or not at all,
+    # at an even and an odd count of tiles. Every P byte is the oracle's, and the run without a
+    # P dump gives the same output.
+    _print_case("control path vanishing", dim, nk)
+    heads, nq, tiles = 257, 17, -(-nk // 128)
+    q, k, v = make_qkv(1, heads, nq, nk, dim, torch.bfloat16, seed=31)
+    for h in range(heads):
+        t = h % (tiles + 1)
+        k[0, h, 128 * t:128 * t + 128] *= 40
+    st = o.prepare(bits(q), bits(k), bits(v), expcast=False, v_smooth=False, dtype="bfloat16")
+    to = _to_dev
+    v8 = to(logical_to_storage(st["v"], vcx.value_token())).view(torch.float8_e4m3fn)
+    args = (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None, False, False,
+            st["output_type"], st["scale"])
+    out, pd = vcx.forward(*args, p_rows=(0, nq))
+    eout, ecodes = o.reference(st, return_codes=True)
+    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+    err, bound = output_bound(out.float().cpu().numpy(), eout)
+    assert np.all(err <= bound), float((err - bound).max())
+    assert torch.equal(vcx.forward(*args), out)
+
+
 def test_control_path_uniform_attention_known_answer_and_end_to_end():
     # scripts/validate_sage_vc.py:161-182: q = k = 0 gives every key p = 2^8.807 (byte 0x7E),
     # so the output is the decoded V mean times 448 / 2^8.807f.
