@@ -26,6 +26,9 @@ struct CallWs {
 
 bool groups(const vcx_call& c) { return c.smooth && c.perm == nullptr; }
 
+// V scales per channel: without smoothing there are no others, whatever the option says.
+bool channel_scales(const vcx_call& c) { return !c.smooth || c.channel_scale; }
+
 CallWs call_ws(const vcx_call& c) {
   const int64_t BH = c.B * c.H, tq = cdiv(c.Nq, 64), tiles = cdiv(c.Nk, kTile);
   size_t off = 0;
@@ -40,7 +43,7 @@ CallWs call_ws(const vcx_call& c) {
   w.v8 = reinterpret_cast<uint8_t*>(take(BH * c.D * tiles * kTile));
   w.qs = reinterpret_cast<float*>(take(sizeof(float) * BH * tq * (c.qk_fp8 ? 1 : 32)));
   w.ks = reinterpret_cast<float*>(take(sizeof(float) * BH * tiles * (c.qk_fp8 ? 1 : 4)));
-  w.vs = reinterpret_cast<float*>(take(sizeof(float) * BH * c.D * (c.channel_scale ? 1 : tiles)));
+  w.vs = reinterpret_cast<float*>(take(sizeof(float) * BH * c.D * (channel_scales(c) ? 1 : tiles)));
   if (c.smooth) w.means = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * BH * tiles * c.D));
   if (groups(c)) w.perm = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * BH * c.Nk));
   // grouping and preparation run one after another on the stream, so they share the scratch
@@ -99,7 +102,7 @@ extern "C" int vcx_attention_call(const vcx_call* c, void* stream) {
                                  static_cast<float>(c->sm_scale), dtype, c->out, c->o_sb, c->o_sh, c->o_sn, nullptr, 0,
                                  0, stream);
   return vcx_attention_fwd(w.q8, w.k8, w.v8, w.qs, w.ks, w.vs, w.means, c->B, c->H, c->Nq, c->Nk, c->D,
-                           static_cast<int>(c->expcast), c->smooth != 0, c->channel_scale != 0,
+                           static_cast<int>(c->expcast), c->smooth != 0, channel_scales(*c),
                            static_cast<float>(c->sm_scale), dtype, c->out, c->o_sb, c->o_sh, c->o_sn, nullptr, 0, 0,
                            stream);
 }

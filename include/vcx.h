@@ -229,7 +229,8 @@ int vcx_attention_fwd_fp8(const uint8_t* q8, const uint8_t* k8, const uint8_t* v
  * workspace (256-byte aligned, vcx_attention_call_bytes bytes: a function of the shape and the
  * options, not of the pointers other than whether perm is null), which is free again once the
  * stream has passed the call. dtype is Q/K/V's and the output's; expcast as for
- * vcx_attention_fwd; perm (nullable int64 [B,H,Nk]) gathers K and V in place of a grouping;
+ * vcx_attention_fwd; channel_scale matters with smooth only (the V scales are per channel
+ * without it); perm (nullable int64 [B,H,Nk]) gathers K and V in place of a grouping;
  * group_mode, clusters and iterations as for vcx_group_values. Every field is 8 bytes.
  * Replaces sageattn_vc's chain of native calls
  * (third_party/sageattention_local/sageattention_local/vc.py:141-197, vc_fp8.py:12-42). */

@@ -123,6 +123,20 @@ def test_invalid_calls_rejected_before_launch():
     assert "aligned" in L.vcx_last_error().decode()
 
 
+def _call_bytes(perm=0, qk_fp8=0, rotate=0, expcast=1, smooth=0, channel_scale=1, clusters=8, iterations=2,
+                group_mode=0, dtype=1, shape=(1, 3, 1000, 1000, 128)):
+    out = ctypes.c_size_t(0)
+    call = vcx._CALL.pack(0, 0, 0, 0, perm, 0, 0, *shape, *(0,) * 12, dtype, qk_fp8, rotate, expcast, smooth,
+                          channel_scale, clusters, iterations, group_mode, 1.0)
+    return vcx.lib().vcx_attention_call_bytes(call, ctypes.byref(out)), out.value
+
+
+def test_one_call_without_smoothing_has_per_channel_scales():
+    # block scales are an option of the smoothing: without it the call is the same one
+    assert _call_bytes(smooth=0, channel_scale=0) == _call_bytes(smooth=0, channel_scale=1)
+    assert _call_bytes(smooth=1, channel_scale=0)[1] > _call_bytes(smooth=1, channel_scale=1)[1]
+
+
 def test_python_binding_refuses_cpu_tensors():
     import torch
     with pytest.raises(vcx.VcxError, match="no CPU fallback"):

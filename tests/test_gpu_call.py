@@ -15,7 +15,7 @@ DEV = torch.device("cuda:0")
 @pytest.mark.parametrize("shape", [(2, 3, 257, 400, 128), (1, 2, 2048, 2048, 64), (1, 1, 1, 1, 128)])
 @pytest.mark.parametrize("layout", ["HND", "NHD"])
 @pytest.mark.parametrize("options", [
-    dict(v_smooth=False), dict(v_smooth=False, kernel_mode="vc9"), dict(v_smooth=False, expcast=False),
+    dict(v_smooth=False), dict(v_smooth=False, v_scale_mode="block"), dict(v_smooth=False, kernel_mode="vc9"), dict(v_smooth=False, expcast=False),
     dict(), dict(v_scale_mode="block"), dict(expcast=False, clusters=16), dict(grouping_mode="legacy", sm_scale=0.2),
 ], ids=lambda o: "_".join("%s-%s" % kv for kv in o.items()) or "default")
 def test_one_call_gives_the_bits_of_its_stages(shape, layout, options):
