@@ -226,6 +226,8 @@ def attention(q, k, v, config=None, *, cache=None, step=0, total_steps=1, reques
                                          layer_id=layer_id)
     import vcx
 
+    if active and pi is None:  # a caller's own cache may smooth the tokens in their given order
+        pi = torch.arange(v.shape[2], device=v.device).expand(v.shape[:3]).contiguous()
     # The ExpCast encode of the reference's default kernel mode: folded without block values.
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     vcx.attention_call(q, k, v, out, perm=pi, rotate=cfg.qk_hadamard,

@@ -55,6 +55,22 @@ def test_one_fp8_call_and_cached_steps_give_the_bits_of_their_stages(expcast):
                                                 affine=expcast and not active))
 
 
+def test_smoothing_without_a_permutation_keeps_the_tokens_order():
+    print("case: smoothing in the given order", flush=True)
+
+    class InOrder(LayoutCache):
+        def layout(self, v, **kwargs):
+            return None, True, False
+
+    q, k, v = (x.to(DEV) for x in make_qkv(1, 3, 300, 1000, 128, torch.bfloat16, seed=9, kind="outlier"))
+    cfg = Config(backend="hip", qk_format="int8", q_block=64, k_quant_block=128, expcast=True, v_smooth=True,
+                 qk_hadamard=False)
+    out, _ = attention(q, k, v, cfg, cache=InOrder(cfg), request_id="r")
+    q8, qs, k8, ks, _ = vcx.prepare_qk(q, k)
+    v8, vs, means = vcx.prepare_v(v, smooth=True)
+    assert torch.equal(out, vcx.forward(q8, k8, v8, qs, ks, vs, means, True, True, 1, 128 ** -0.5))
+
+
 def test_one_call_under_capture_replays_to_the_same_bits():
     print("case: one call captured", flush=True)
     q, k, v = (x.to(DEV) for x in make_qkv(1, 2, 300, 700, 128, torch.bfloat16, seed=7, kind="outlier"))
