@@ -137,6 +137,26 @@ def test_one_call_without_smoothing_has_per_channel_scales():
     assert _call_bytes(smooth=1, channel_scale=0)[1] > _call_bytes(smooth=1, channel_scale=1)[1]
 
 
+@pytest.mark.parametrize("name,shape", [("q", (2, 3, 5, 64)), ("q", (1, 3, 5, 128)), ("k", (1, 2, 7, 64)), ("k", (1, 3, 8, 64)),
+                                        ("k", (3, 7, 64)), ("v", (1, 3, 6, 64)), ("v", (1, 3, 7, 128)),
+                                        ("out", (1, 3, 4, 64)), ("out", (1, 3, 5, 128)), ("out", (3, 5, 64))])
+def test_one_call_refuses_tensors_of_other_shapes(name, shape):
+    # refused before the tensors' device is looked at, as they would be read past their end
+    import torch
+    t = {"q": (1, 3, 5, 64), "k": (1, 3, 7, 64), "v": (1, 3, 7, 64), "out": (1, 3, 5, 64), name: shape}
+    t = {n: torch.zeros(x, dtype=torch.float16) for n, x in t.items()}
+    with pytest.raises(vcx.VcxError, match="must be"):
+        vcx.attention_call(**t, expcast=2, smooth=False, scale=0.125)
+
+
+@pytest.mark.parametrize("name", ["q", "k", "v", "out"])
+def test_one_call_refuses_other_types(name):
+    import torch
+    t = {n: torch.zeros(1, 3, 5, 64, dtype=torch.bfloat16 if n == name else torch.float16) for n in ("q", "k", "v", "out")}
+    with pytest.raises(vcx.VcxError, match="float16/bfloat16"):
+        vcx.attention_call(**t, expcast=2, smooth=False, scale=0.125)
+
+
 def test_python_binding_refuses_cpu_tensors():
     import torch
     with pytest.raises(vcx.VcxError, match="no CPU fallback"):
