@@ -60,8 +60,13 @@ int check_call(const vcx_call* c) {
   VCX_REQUIRE(c->D == 64 || c->D == 128, "D must be 64 or 128");
   VCX_REQUIRE(c->B <= 65535 && c->H <= 65535 && c->B * c->H <= 65535, "B*H exceeds 65535");
   VCX_REQUIRE(c->Nq < (int64_t(1) << 30) && c->Nk < (int64_t(1) << 30), "sequence too long");
-  VCX_REQUIRE(!c->smooth || c->perm != nullptr || (c->clusters >= 1 && c->clusters <= 256),
-              "clusters must be in [1, 256]");
+  // the stages take these as int: nothing may be lost on the way
+  VCX_REQUIRE(c->dtype == VCX_FLOAT16 || c->dtype == VCX_BFLOAT16, "dtype must be float16 or bfloat16");
+  VCX_REQUIRE(c->expcast >= 0 && c->expcast <= 2, "expcast must be 0, 1 or 2");
+  VCX_REQUIRE(!groups(*c) || (c->clusters >= 1 && c->clusters <= 256 && c->iterations >= 1 && c->iterations <= 100),
+              "clusters must be in [1, 256] and iterations in [1, 100]");
+  VCX_REQUIRE(!groups(*c) || c->group_mode == VCX_GROUP_AUTO || c->group_mode == VCX_GROUP_GENERAL,
+              "mode must be VCX_GROUP_AUTO or VCX_GROUP_GENERAL");
   VCX_REQUIRE(!c->qk_fp8 || (!c->smooth && !c->rotate && c->perm == nullptr),
               "FP8 QK takes no V smoothing, rotation or permutation");
   return VCX_OK;

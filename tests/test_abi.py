@@ -137,6 +137,16 @@ def test_one_call_without_smoothing_has_per_channel_scales():
     assert _call_bytes(smooth=1, channel_scale=0)[1] > _call_bytes(smooth=1, channel_scale=1)[1]
 
 
+@pytest.mark.parametrize("option,value", [("dtype", 2**32), ("dtype", 2), ("expcast", 2**32 + 2), ("expcast", 3),
+                                          ("iterations", 2**32 + 2), ("iterations", 0), ("clusters", 257),
+                                          ("group_mode", 2**32), ("group_mode", 2)])
+def test_one_call_loses_no_part_of_an_option(option, value):
+    # the call's fields are 64 bits wide, the stages' arguments 32
+    assert _call_bytes(smooth=1)[0] == 0
+    rc, _ = _call_bytes(**{"smooth": 1, option: value})
+    assert rc == 1 and option.split("_")[-1] in vcx.lib().vcx_last_error().decode()
+
+
 @pytest.mark.parametrize("name,shape", [("q", (2, 3, 5, 64)), ("q", (1, 3, 5, 128)), ("k", (1, 2, 7, 64)), ("k", (1, 3, 8, 64)),
                                         ("k", (3, 7, 64)), ("v", (1, 3, 6, 64)), ("v", (1, 3, 7, 128)),
                                         ("out", (1, 3, 4, 64)), ("out", (1, 3, 5, 128)), ("out", (3, 5, 64))])
