@@ -6,11 +6,10 @@
 
 namespace vcx {
 
-size_t ws_prepare_qk(int64_t BH, int64_t N, int64_t D);
 size_t ws_prepare_v(int64_t BH, int64_t N, int64_t D);
 size_t ws_group(int64_t BH, int64_t N, int64_t D, int clusters);
 int prepare_together(const vcx_call& c, const int64_t* perm, void* q8, float* qs, void* k8, float* ks, uint8_t* v8,
-                     float* vs, uint16_t* means, void* scratch, void* stream);
+                     float* vs, uint16_t* means, double* ksum, float* km, void* v_scratch, void* stream);
 
 namespace {
 
@@ -20,8 +19,9 @@ struct CallWs {
   float *qs, *ks, *vs;
   uint16_t* means;
   int64_t* perm;
-  void* scratch;
-  size_t scratch_bytes, bytes;
+  float* km;
+  void *v_scratch, *group_scratch;
+  size_t group_bytes, bytes;
 };
 
 bool groups(const vcx_call& c) { return c.smooth && c.perm == nullptr; }
@@ -29,6 +29,9 @@ bool groups(const vcx_call& c) { return c.smooth && c.perm == nullptr; }
 // V scales per channel: without smoothing there are no others, whatever the option says.
 bool channel_scales(const vcx_call& c) { return !c.smooth || c.channel_scale; }
 
+// Two places serve twice, as the stages run one after another on the stream: the grouping's scratch
+// lies over all that is written after it, and K's tile sums (8 bytes per channel and tile), which
+// the Q launch reads last, over the V payload (128 bytes), which the launch after that writes.
 CallWs call_ws(const vcx_call& c) {
   const int64_t BH = c.B * c.H, tq = cdiv(c.Nq, 64), tiles = cdiv(c.Nk, kTile);
   size_t off = 0;
@@ -38,6 +41,8 @@ CallWs call_ws(const vcx_call& c) {
     return p;
   };
   CallWs w{};
+  if (groups(c)) w.perm = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * BH * c.Nk));
+  const size_t shared = off;
   w.q8 = reinterpret_cast<int8_t*>(take(BH * c.Nq * c.D));
   w.k8 = reinterpret_cast<int8_t*>(take(BH * c.Nk * c.D));
   w.v8 = reinterpret_cast<uint8_t*>(take(BH * c.D * tiles * kTile));
@@ -45,11 +50,13 @@ CallWs call_ws(const vcx_call& c) {
   w.ks = reinterpret_cast<float*>(take(sizeof(float) * BH * tiles * (c.qk_fp8 ? 1 : 4)));
   w.vs = reinterpret_cast<float*>(take(sizeof(float) * BH * c.D * (channel_scales(c) ? 1 : tiles)));
   if (c.smooth) w.means = reinterpret_cast<uint16_t*>(take(sizeof(uint16_t) * BH * tiles * c.D));
-  if (groups(c)) w.perm = reinterpret_cast<int64_t*>(take(sizeof(int64_t) * BH * c.Nk));
-  // grouping and preparation run one after another on the stream, so they share the scratch
-  w.scratch_bytes = ws_prepare_qk(BH, c.Nk, c.D) + ws_prepare_v(BH, c.Nk, c.D);
-  if (groups(c)) w.scratch_bytes = std::max(w.scratch_bytes, ws_group(BH, c.Nk, c.D, static_cast<int>(c.clusters)));
-  w.scratch = take(w.scratch_bytes);
+  w.km = reinterpret_cast<float*>(take(sizeof(float) * BH * c.D));
+  w.v_scratch = take(ws_prepare_v(BH, c.Nk, c.D));
+  if (groups(c)) {
+    w.group_scratch = static_cast<char*>(c.workspace) + shared;
+    w.group_bytes = ws_group(BH, c.Nk, c.D, static_cast<int>(c.clusters));
+    off = std::max(off, shared + w.group_bytes);
+  }
   w.bytes = off;
   return w;
 }
@@ -96,11 +103,13 @@ extern "C" int vcx_attention_call(const vcx_call* c, void* stream) {
     if (int rc = vcx_group_values(c->v, dtype, c->B, c->H, c->Nk, c->D, c->v_sb, c->v_sh, c->v_sn,
                                   static_cast<int>(c->clusters), static_cast<int>(c->iterations),
                                   static_cast<int>(c->group_mode), nullptr, w.perm, nullptr, nullptr, nullptr,
-                                  w.scratch, w.scratch_bytes, stream))
+                                  w.group_scratch, w.group_bytes, stream))
       return rc;
     perm = w.perm;
   }
-  if (int rc = prepare_together(*c, perm, w.q8, w.qs, w.k8, w.ks, w.v8, w.vs, w.means, w.scratch, stream)) return rc;
+  double* ksum = reinterpret_cast<double*>(w.v8);
+  if (int rc = prepare_together(*c, perm, w.q8, w.qs, w.k8, w.ks, w.v8, w.vs, w.means, ksum, w.km, w.v_scratch, stream))
+    return rc;
   if (c->qk_fp8)
     return vcx_attention_fwd_fp8(reinterpret_cast<uint8_t*>(w.q8), reinterpret_cast<uint8_t*>(w.k8), w.v8, w.qs, w.ks,
                                  w.vs, c->B, c->H, c->Nq, c->Nk, c->D, static_cast<int>(c->expcast),

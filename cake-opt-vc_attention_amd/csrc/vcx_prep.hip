@@ -1013,11 +1013,12 @@ extern "C" int vcx_prepare_qk_int8_rotated(const void* q, const void* k, int dty
 }
 
 // Q, K and V of one call in three launches. Outputs and results are those of
-// vcx_prepare_qk_int8(_rotated) or vcx_prepare_qk_fp8, and vcx_prepare_v_fp8. The scratch holds
-// both stages' workspaces.
+// vcx_prepare_qk_int8(_rotated) or vcx_prepare_qk_fp8, and vcx_prepare_v_fp8. ksum: K's tile sums
+// (may lie over v8: the first launch writes them, the second reads them, the third writes v8);
+// km: K's mean; v_scratch: vcx_prepare_v_fp8's workspace.
 namespace vcx {
 int prepare_together(const vcx_call& c, const int64_t* perm, void* q8, float* qs, void* k8, float* ks, uint8_t* v8,
-                     float* vs, uint16_t* means, void* scratch, void* stream) {
+                     float* vs, uint16_t* means, double* ksum, float* km, void* v_scratch, void* stream) {
   if (int rc = check_shape(c.B, c.H, c.Nq, c.D)) return rc;
   if (int rc = check_shape(c.B, c.H, c.Nk, c.D)) return rc;
   VCX_REQUIRE(c.dtype == VCX_FLOAT16 || c.dtype == VCX_BFLOAT16, "dtype must be float16 or bfloat16");
@@ -1026,10 +1027,7 @@ int prepare_together(const vcx_call& c, const int64_t* perm, void* q8, float* qs
   if (int rc = check_input("v", c.v, c.B, c.H, c.Nk, c.D, c.v_sb, c.v_sh, c.v_sn)) return rc;
   VCX_REQUIRE(aligned(perm, 8), "perm misaligned");
   const int64_t BH = c.B * c.H, tiles = cdiv(c.Nk, kTile);
-  auto* ws = static_cast<char*>(scratch);
-  double* ksum = reinterpret_cast<double*>(ws);
-  float* km = reinterpret_cast<float*>(ws + align_up(sizeof(double) * BH * tiles * c.D));
-  ws += ws_prepare_qk(BH, c.Nk, c.D);
+  auto* ws = static_cast<char*>(v_scratch);
   const size_t slice = align_up(sizeof(float) * BH * tiles * c.D);
   float* a0 = reinterpret_cast<float*>(ws);
   float* a1 = reinterpret_cast<float*>(ws + slice);

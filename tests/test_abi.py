@@ -137,6 +137,23 @@ def test_one_call_without_smoothing_has_per_channel_scales():
     assert _call_bytes(smooth=1, channel_scale=0)[1] > _call_bytes(smooth=1, channel_scale=1)[1]
 
 
+@pytest.mark.parametrize("shape", [(1, 28, 75482, 75482, 128), (2, 3, 257, 4000, 64), (1, 1, 1, 1, 128)])
+@pytest.mark.parametrize("smooth,channel,fp8", [(0, 1, 0), (1, 1, 0), (1, 0, 0), (0, 1, 1)])
+def test_one_call_needs_no_more_memory_than_its_stages(shape, smooth, channel, fp8):
+    B, H, Nq, Nk, D = shape
+    BH, tq, tiles = B * H, (Nq + 63) // 64, (Nk + 127) // 128
+    got = _call_bytes(smooth=smooth, channel_scale=channel, qk_fp8=fp8, shape=shape)[1]
+    ws = [vcx.workspace_bytes(op, B, H, Nk, D) for op in (vcx.WS_PREPARE_QK, vcx.WS_PREPARE_V, vcx.WS_GROUP)]
+    perm = 8 * BH * Nk if smooth else 0
+    qk = BH * (Nq + Nk) * D + 4 * BH * ((tq + tiles) if fp8 else (32 * tq + 4 * tiles)) + 4 * BH * D  # mean
+    v = BH * D * 128 * tiles + 4 * BH * D * (1 if channel else tiles) + (2 * BH * tiles * D if smooth else 0)
+    # grouping; Q/K with their scratch; then V with its own
+    stages = max(perm + ws[2] if smooth else 0, perm + qk + ws[0], perm + qk + v + ws[1])
+    assert got <= stages + 10 * 256  # every piece is rounded up to 256 bytes
+    if smooth:
+        assert got >= perm + max(ws[2], qk + v + ws[1])
+
+
 @pytest.mark.parametrize("option,value", [("dtype", 2**32), ("dtype", 2), ("expcast", 2**32 + 2), ("expcast", 3),
                                           ("iterations", 2**32 + 2), ("iterations", 0), ("clusters", 257),
                                           ("group_mode", 2**32), ("group_mode", 2)])
