@@ -76,21 +76,24 @@ __device__ __forceinline__ void body_tiles(W& w, const LD& ld, const AttnArgs& a
   for (; t + 2 <= end; t += 2) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if constexpr (!W::kSpread) ld.issue(t + 1, lds1, lds1 + KB, meta1);
     w.template tile<false, PRE>(a, t, lds0, lds0 + KB, meta0, [&](int i) {
-      if (i < LD::kParts) ld.part(i, t + 1, lds1, lds1 + KB, meta1);
+      if (W::kSpread && i < LD::kParts) ld.part(i, t + 1, lds1, lds1 + KB, meta1);
     });
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if constexpr (!W::kSpread) ld.issue(t + 2, lds0, lds0 + KB, meta0);
     w.template tile<false, PRE>(a, t + 1, lds1, lds1 + KB, meta1, [&](int i) {
-      if (i < LD::kParts) ld.part(i, t + 2, lds0, lds0 + KB, meta0);
+      if (W::kSpread && i < LD::kParts) ld.part(i, t + 2, lds0, lds0 + KB, meta0);
     });
     if constexpr (kLeaves) end = wave_any(w.wide != 0) ? 0 : body;
   }
   if (kLeaves ? t + 1 == body : t < body) {  // odd count of body tiles: one more from buffer 0, last tile lands in buffer 1
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
+    if constexpr (!W::kSpread) ld.issue(t + 1, lds1, lds1 + KB, meta1);
     w.template tile<false, PRE>(a, t, lds0, lds0 + KB, meta0, [&](int i) {
-      if (i < LD::kParts) ld.part(i, t + 1, lds1, lds1 + KB, meta1);
+      if (W::kSpread && i < LD::kParts) ld.part(i, t + 1, lds1, lds1 + KB, meta1);
     });
     ++t;
   }

@@ -265,6 +265,12 @@ struct Wave {
   static constexpr bool IB = QF == 0 && (PM == 2 || (PM == 1 && D == 128 && VM == 1) ||
                                          (PM == 0 && D == 128 && !(VM == 2 && DUMP)));
   static constexpr int kD = D, kPM = PM;
+  // Whether the next tile's loads are spread over the QK steps (see tile) or all issued before
+  // them. A D64 tile has half the loads and half the MFMA time: spread, the last load lands too
+  // late for a tile without block values, the shortest one. Same box, us, issued first / spread: FP8
+  // [1,2,40001,64] 653 / 706, [1,24,16001,64] 1102 / 1169, [1,16,8192,64] unfused 253 / 259, control 328 /
+  // 338; INT8 [1,24,16001,64] 932 / 939, [2,16,4097,64] 107.3 / 107.7.
+  static constexpr bool kSpread = D == 128 || VM > 0;
   static constexpr int DS = D / 64;  // 64-deep QK steps
   static constexpr int CB = D / 16;  // 16-channel output blocks
   static constexpr bool SMOOTH = VM >= 1, BSCALE = VM == 2;
