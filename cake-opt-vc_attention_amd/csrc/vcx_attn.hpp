@@ -271,6 +271,10 @@ struct Wave {
   // [1,2,40001,64] 653 / 706, [1,24,16001,64] 1102 / 1169, [1,16,8192,64] unfused 253 / 259, control 328 /
   // 338; INT8 [1,24,16001,64] 932 / 939, [2,16,4097,64] 107.3 / 107.7.
   static constexpr bool kSpread = D == 128 || VM > 0;
+  // Control path: whether the copy of the loop without small probabilities pays (see bytes). At
+  // D128 with per-block V scales two copies spill (527 scalars and 178 vector registers against
+  // 296 and 170 in one): [1,16,8192,128] 1194 us with both, 800 us with the general one.
+  static constexpr bool kCheapTest = D == 64 || VM < 2;
   static constexpr int DS = D / 64;  // 64-deep QK steps
   static constexpr int CB = D / 16;  // 16-channel output blocks
   static constexpr bool SMOOTH = VM >= 1, BSCALE = VM == 2;
