@@ -327,67 +327,6 @@ template __global__ void attn_kernel<128, 0, false, 1, 0, 1>(AttnArgs);
 template __global__ void attn_kernel<128, 0, true, 0, 0, 1>(AttnArgs);
 template __global__ void attn_kernel<128, 0, true, 1, 0, 1>(AttnArgs);
 
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
-
 // Makespan, in units of one 128-row block's time, of one XCD's block list on S slots served
 // in list order, each block to the slot that frees first: n - k full blocks, then 2k halves
 // of relative length h.
