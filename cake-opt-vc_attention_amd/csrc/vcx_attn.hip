@@ -457,8 +457,9 @@ extern "C" int vcx_attention_fwd(const int8_t* q8, const int8_t* k8, const uint8
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool dump = p_dump != nullptr;
   a.out_bf16 = out_dtype == VCX_BFLOAT16;
-  if (const int groups = piece_groups(B * H, Nq, D))
-    return launch_pieces(a, B * H, D, groups, block_values ? (channel_scale ? 1 : 2) : 0, expcast, 0, st);
+  const int vm = block_values ? (channel_scale ? 1 : 2) : 0;
+  if (const int groups = piece_groups(B * H, Nq, a.tiles, D, vm, expcast, 0))
+    return launch_pieces(a, B * H, D, groups, vm, expcast, 0, st);
   if (D == 128) {
     if (!block_values) return launch_mode<128, 0>(a, dump, out_dtype, expcast, st);
     return channel_scale ? launch_mode<128, 1>(a, dump, out_dtype, expcast, st)
@@ -494,7 +495,8 @@ extern "C" int vcx_attention_fwd_fp8(const uint8_t* q8, const uint8_t* k8, const
   hipStream_t st = static_cast<hipStream_t>(stream);
   const bool dump = p_dump != nullptr;
   a.out_bf16 = out_dtype == VCX_BFLOAT16;
-  if (const int groups = piece_groups(B * H, Nq, D)) return launch_pieces(a, B * H, D, groups, 0, expcast, 1, st);
+  if (const int groups = piece_groups(B * H, Nq, a.tiles, D, 0, expcast, 1))
+    return launch_pieces(a, B * H, D, groups, 0, expcast, 1, st);
   return D == 128 ? launch_mode<128, 0, 1>(a, dump, out_dtype, expcast, st)
                   : launch_mode<64, 0, 1>(a, dump, out_dtype, expcast, st);
 }

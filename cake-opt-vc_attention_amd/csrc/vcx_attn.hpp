@@ -29,7 +29,7 @@ struct AttnArgs {
 };
 
 // vcx_attn_piece.hip
-int piece_groups(int64_t BH, int64_t Nq, int64_t D);
+int piece_groups(int64_t BH, int64_t Nq, int64_t tiles, int64_t D, int vm, int mode, int qf);
 int launch_pieces(const AttnArgs& a, int64_t BH, int64_t D, int groups, int vm, int mode, int qf, hipStream_t st);
 
 namespace {

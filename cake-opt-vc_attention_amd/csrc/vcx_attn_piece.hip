@@ -384,13 +384,36 @@ int launch_values(const AttnArgs& a, int64_t BH, int groups, int vm, int mode, i
 //   [1,8,2048 x 8192,128]           59.2    - / 66.4 (512 pieces) / 54.0
 //   [1,4,1024 x 8192,64] smoothing  47.7  20.7 / 28.8 / 44.9
 //   [1,8,2048 x 8192,64] smoothing  48.5    - / 55.6 (512 pieces) / 45.7
-int piece_groups(int64_t BH, int64_t Nq, int64_t D) {
+// And 0 where the keys are too few for the splits to pay, as a piece starts and ends more slowly
+// than a block (pieces' time over attn_kernel's in replayed graphs, by key tiles; the folded
+// encode of INT8 scores / the other modes):
+//   1 or 2 groups, D64   1: 1.03-1.07 / 1.26-1.46, 2: 0.93-0.98 / 1.04-1.26, 3: 0.90 / 0.89-1.14,
+//                        4: 0.83 / 0.76-1.01, 8: 0.70-0.83 / 0.57-0.89
+//   2 groups, D128       1: 1.00 / 1.18-1.28, 2: 0.91 / 0.93-1.11, 4: 0.82 / 0.77-0.96, 8: 0.78 / 0.70-0.85
+// With four groups the two splits stand against attn_kernel's 64-row blocks, which the same rows
+// fill the chip with if the 128-row blocks deal out evenly over the XCDs (tail_split halves equally
+// many on each). There the splits pay late, or not at all at D128 (64 tiles: folded 1.00, control
+// 1.04-1.09), but for per-block V scales (8 tiles 0.91-0.99, 64 tiles 0.73-0.89) and the folded encode
+// of D64 or FP8 scores (8 tiles 0.89-0.98, 64 tiles 0.68-0.97); the rest of D64: 8 tiles 1.00-1.10, 24 tiles
+// 0.91-1.00, 64 tiles 0.89-1.04; at D128 without the control path 256 tiles 0.80-1.02, the less the
+// more heads (K and V past the caches). Where they don't, attn_kernel keeps 128-row blocks, and pieces take
+// 0.55-0.73 of its time at [1,9,1100 x 1024..8192].
+// Up to eight pieces, one per XCD, each pays for its own code's way to the caches, which is
+// shorter for pieces: [1,1,64 x 77,128] 6.5-7.5 against 9.6-10.6 us, [1,1,64 x 256,64] 5.8-6.4 against 8.3-9.0.
+int piece_groups(int64_t BH, int64_t Nq, int64_t tiles, int64_t D, int vm, int mode, int qf) {
   int dev = 0, cus = 0;
   if (hipGetDevice(&dev) != hipSuccess ||
       hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
     return 0;
-  for (int rg = D == 128 ? 2 : 1; rg <= 4; rg *= 2)
-    if (BH * cdiv(Nq, 16 * rg) <= cus) return rg;
+  for (int rg = D == 128 ? 2 : 1; rg <= 4; rg *= 2) {
+    const int64_t pieces = BH * cdiv(Nq, 16 * rg);
+    if (pieces > cus) continue;
+    if (pieces <= 8) return tiles >= (D == 128 ? 1 : 2) ? rg : 0;
+    const bool folded = mode == 2;
+    if (rg < 4 || BH * cdiv(Nq, kRowsPerBlock) % 8 != 0) return tiles >= (folded && !qf ? 2 : 4) ? rg : 0;
+    if (vm == 2 || (folded && (D == 64 || qf))) return tiles >= 8 ? rg : 0;
+    return D == 64 ? (tiles >= 24 ? rg : 0) : (mode != 0 && tiles >= 192 ? rg : 0);
+  }
   return 0;
 }
 
