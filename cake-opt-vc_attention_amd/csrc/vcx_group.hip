@@ -775,23 +775,26 @@ __global__ __launch_bounds__(128) void grp_update_kernel(float* centers, double*
   }
 }
 
-// General schedule. grid (B*H, count, D / 32), 1024 threads: the new center of one cluster for
+// General schedule. grid (B*H, count, D / 32), THREADS threads: the new center of one cluster for
 // 32 channels. Cluster c's tokens of tile t are perm[offsets[t][c] .. + pcnt[t][c]), ascending.
 // Only the tile partials are chained (over tiles, in order); the partials themselves are
-// independent, so 64 groups of 16 lanes (two adjacent channels each) form those of up to
-// kUpdateTiles tiles at once, and one thread per channel then adds them from LDS in tile
+// independent, so THREADS / 16 groups of 16 lanes (two adjacent channels each) form those of
+// up to kTiles tiles at once, and one thread per channel then adds them from LDS in tile
 // order. A tile without the cluster adds +0.0, which leaves the sum unchanged (it starts at
 // +0.0 and is never -0.0). The kernel is bound by the load round trips of a partial (offset,
 // token, row), of which 1024 threads keep enough in flight: at [1,7,37741,128] fp16 with 16
 // clusters 2044 us with one thread per channel walking the whole token list, 47 us with
-// this split.
-constexpr int kUpdateThreads = 1024, kUpdateChannels = 32, kUpdateTiles = 256;
-template <int DT>
-__global__ __launch_bounds__(kUpdateThreads) void grp_update_sorted_kernel(
+// this split. Few tiles leave most of these threads without a list, and of many clusters' blocks
+// few fit: 64 threads up to 4 tiles, 256 up to 16. Whole grouping with 256 clusters, us, one
+// thread per channel / 1024 threads / this: [1,28,256,128] 836 / 893 / 795, [1,28,2048,128] 1742 /
+// 1723 / 1629.
+constexpr int kUpdateChannels = 32;
+template <int DT, int THREADS>
+__global__ __launch_bounds__(THREADS) void grp_update_sorted_kernel(
     const void* v, int64_t H, int64_t n, int64_t sb, int64_t sh, int64_t sn, int count, int CS, const int64_t* perm,
     const int64_t* offsets, const int32_t* pcnt, int64_t tiles, int D, float* centers, double* centers64) {
-  constexpr int kPairs = kUpdateChannels / 2, kLists = kUpdateThreads / kPairs, kRuns = kUpdateTiles / kLists;
-  __shared__ double2 part[kUpdateTiles * kPairs];
+  constexpr int kPairs = kUpdateChannels / 2, kLists = THREADS / kPairs, kRuns = 4, kTiles = kLists * kRuns;
+  __shared__ double2 part[kTiles * kPairs];
   const int64_t bh = blockIdx.x;
   const int c = blockIdx.y, tid = threadIdx.x, pair = tid % kPairs, list = tid / kPairs;
   const int d0 = blockIdx.z * kUpdateChannels;
@@ -800,7 +803,7 @@ __global__ __launch_bounds__(kUpdateThreads) void grp_update_sorted_kernel(
   const int32_t* cnt = pcnt + bh * tiles * CS + c;
   const int64_t* p = perm + bh * n;
   double s = 0.0;  // threads below kUpdateChannels: their channel's sum
-  for (int64_t t0 = 0; t0 < tiles; t0 += kUpdateTiles) {
+  for (int64_t t0 = 0; t0 < tiles; t0 += kTiles) {
     int64_t begin[kRuns];
     int num[kRuns];
 #pragma unroll
@@ -832,7 +835,7 @@ __global__ __launch_bounds__(kUpdateThreads) void grp_update_sorted_kernel(
     __syncthreads();
     if (tid < kUpdateChannels) {
       const double* col = reinterpret_cast<const double*>(part) + tid;
-      const int m = static_cast<int>(tiles - t0 < kUpdateTiles ? tiles - t0 : kUpdateTiles);
+      const int m = static_cast<int>(tiles - t0 < kTiles ? tiles - t0 : kTiles);
 #pragma unroll 16
       for (int t = 0; t < m; ++t) s = __dadd_rn(s, col[t * kUpdateChannels]);
     }
@@ -1175,8 +1178,14 @@ extern "C" int vcx_group_values(const void* v, int dtype, int64_t B, int64_t H, 
         if (last && centers)
           if (int rc = copy_centers(centers)) return rc;
         if (update) {
-          grp_update_sorted_kernel<DT><<<dim3(BH, count, DD / kUpdateChannels), kUpdateThreads, 0, st>>>(
-              v, H, N, v_sb, v_sh, v_sn, count, CS, perm, ws.offsets, ws.pcnt, tiles, DD, ws.centers, ws.centers64);
+          auto sorted = [&](auto threads) {
+            constexpr int T = decltype(threads)::value;
+            grp_update_sorted_kernel<DT, T><<<dim3(BH, count, DD / kUpdateChannels), T, 0, st>>>(
+                v, H, N, v_sb, v_sh, v_sn, count, CS, perm, ws.offsets, ws.pcnt, tiles, DD, ws.centers, ws.centers64);
+          };
+          if (tiles <= 4) sorted(std::integral_constant<int, 64>());
+          else if (tiles <= 16) sorted(std::integral_constant<int, 256>());
+          else sorted(std::integral_constant<int, 1024>());
           VCX_LAUNCHED("grp_update_sorted_kernel");
         }
       }

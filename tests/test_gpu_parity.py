@@ -347,7 +347,9 @@ def test_grouping_sort_of_few_labels(n, clusters):
 
 
 @pytest.mark.parametrize("dim,dtype", [(64, torch.float16), (128, torch.bfloat16)])
-@pytest.mark.parametrize("n,clusters", [(256 * 128, 9), (256 * 128 + 1, 9), (512 * 128 - 1, 200)])
+@pytest.mark.parametrize("n,clusters", [(256 * 128, 9), (256 * 128 + 1, 9), (512 * 128 - 1, 200),
+                                        # 64, 256 and 1024 threads
+                                        (4 * 128, 9), (4 * 128 + 1, 16), (16 * 128, 40), (16 * 128 + 1, 9)])
 def test_grouping_sorted_update_at_its_tile_chunks(dim, dtype, n, clusters):
     # The general schedule's update forms the partials of 256 tiles at a time: exactly one full
     # chunk, one token past it, and two chunks with a partial last tile and clusters that many
