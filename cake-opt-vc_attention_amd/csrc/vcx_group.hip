@@ -203,14 +203,19 @@ __device__ void wave_rows_b64(const uint16_t* xs, int row0, uint64_t& open, cons
 // which the assignment reads with wave-uniform (scalar) loads. Slots are CS per head
 // (CS = 8 for the fused schedule, count rounded up to 8 for the general one); slots at or
 // past count hold zeros. Initial values: centers_in [BH][count][D], else V[ids].
-// grid (B*H, CS), D threads: one slot per block (one block per head walked its slots one after
-// another: 5.2 against 3.3 us at two heads, 8.4 against 4.8 us at 28).
+// grid (B*H rounded up to the 8 XCDs, CS), D threads: one slot per block (one block per head
+// walked its slots one after another: 5.2 against 3.3 us at two heads, 8.4 against 4.8 us at 28).
+// A head's slots lie on one XCD (blocks are dealt out in turn), that of its first tile's
+// assignment: with a grid of B*H they lay on all, and the assignment of a single tile read
+// its centers from memory ([1,1,100,128], 64
+// clusters, the whole grouping 196 us so, 175 us now).
 template <int DT>
-__global__ __launch_bounds__(128) void grp_init_kernel(const void* v, int64_t H, int64_t sb, int64_t sh, int64_t sn,
-                                                       Ids ids, int count, int CS, int D, const float* centers_in,
+__global__ __launch_bounds__(128) void grp_init_kernel(const void* v, int64_t BH, int64_t H, int64_t sb, int64_t sh,
+                                                       int64_t sn, Ids ids, int count, int CS, int D, const float* centers_in,
                                                        float* centers, double* centers64, CenterForms forms) {
   __shared__ double red[2];
   const int64_t bh = blockIdx.x;
+  if (bh >= BH) return;
   const int c = blockIdx.y, d = threadIdx.x;
   const int64_t slot = bh * CS + c;
   float x = 0.0f;
@@ -1150,7 +1155,7 @@ extern "C" int vcx_group_values(const void* v, int dtype, int64_t B, int64_t H, 
       VCX_LAUNCHED("grp_scatter_kernel");
       return VCX_OK;
     };
-    grp_init_kernel<DT><<<dim3(BH, CS), DD, 0, st>>>(v, H, v_sb, v_sh, v_sn, ids, count, CS, DD, centers_in,
+    grp_init_kernel<DT><<<dim3(8 * cdiv(BH, 8), CS), DD, 0, st>>>(v, BH, H, v_sb, v_sh, v_sn, ids, count, CS, DD, centers_in,
                                                   ws.centers, ws.centers64,
                                                   DT == VCX_BFLOAT16 ? ws.forms : CenterForms{});
     VCX_LAUNCHED("grp_init_kernel");
