@@ -487,6 +487,10 @@ __device__ inline void load_quad(const void* x, int64_t i, float (&v)[4]) {
 template <bool WIDE, bool MEAN>
 constexpr int kPreRows = WIDE || MEAN ? 4 : 1;
 
+// Blocks of pre_rows_kernel along the grid's x; more of them go on along z, as the threads along
+// one axis stay below 2^32.
+constexpr int64_t kRowsGridX = int64_t(1) << 22;
+
 // grid (tiles, B*H), D threads: binary64 sum of channel d over the tile's keys in key order.
 template <int DT>
 __global__ __launch_bounds__(128) void pre_tile_sum_kernel(const void* x, int64_t H, int64_t n, int64_t sb,
@@ -554,8 +558,9 @@ template <int DT, int W, bool ROT, bool WIDE, bool KM, int NR>
 __global__ __launch_bounds__(kThreads) void pre_rows_kernel(const void* x, int64_t H, int64_t n, int D, int64_t sb,
                                                             int64_t sh, int64_t sn, const float* mean, float* out,
                                                             float norm, KMeanArgs kma) {
+  int64_t blk = blockIdx.z * kRowsGridX + blockIdx.x;
   if constexpr (KM) {
-    if (blockIdx.x == 0) {
+    if (blk-- == 0) {
       if (static_cast<int>(threadIdx.x) < D)
         k_mean_body<VCX_BFLOAT16, true>(kma.sums, kma.tiles, kma.n, D, kma.km, nullptr, blockIdx.y, threadIdx.x);
       return;
@@ -564,7 +569,7 @@ __global__ __launch_bounds__(kThreads) void pre_rows_kernel(const void* x, int64
   constexpr int L = W < 16 ? W : 16, CPT = W / L, RPB = kThreads / L * NR;
   constexpr bool SPLIT = W == 128;
   const int tid = threadIdx.x, c = tid % L;
-  const int64_t bh = blockIdx.y, r0 = static_cast<int64_t>(KM ? blockIdx.x - 1 : blockIdx.x) * RPB + tid / L;
+  const int64_t bh = blockIdx.y, r0 = blk * RPB + tid / L;
   const int64_t head = (bh / H) * sb + (bh % H) * sh;
   auto channel = [&](int j) { return SPLIT ? 4 * c + (j & 3) + 64 * (j >> 2) : c * CPT + j; };
   float v[NR][CPT];
@@ -1273,9 +1278,10 @@ int preprocess_launch(const void* q, const void* k, int64_t BH, int64_t H, int64
                     float* out) {
       constexpr bool KM = decltype(km)::value;
       constexpr int NR = decltype(nr)::value, RPB = kThreads / L * NR;
+      const int64_t blocks = cdiv(n, RPB) + (KM ? 1 : 0), gx = std::min(blocks, kRowsGridX);
       pre_rows_kernel<DT, WW, ROT, decltype(wide)::value, KM, NR>
-          <<<dim3(static_cast<unsigned>(cdiv(n, RPB) + (KM ? 1 : 0)), static_cast<unsigned>(BH)), kThreads, 0, st>>>(
-              x, H, n, static_cast<int>(D), sb, sh, sn, mu, out, norm, kma);
+          <<<dim3(static_cast<unsigned>(gx), static_cast<unsigned>(BH), static_cast<unsigned>(cdiv(blocks, gx))), kThreads,
+             0, st>>>(x, H, n, static_cast<int>(D), sb, sh, sn, mu, out, norm, kma);
     };
     const float* none = nullptr;
     auto launch = [&](bool wide, auto km, auto centre, auto... args) {

@@ -107,6 +107,20 @@ def test_preprocess_qk_bit_exact_and_matrix_oracle(dim, dtype, k_smooth, rotate)
     torch.testing.assert_close(kd.cpu(), k, atol=0, rtol=0)
 
 
+def test_preprocess_qk_more_rows_than_one_grid_axis_holds():
+    # 2^28 + 3 rows in blocks of 16 are more than 2^32 threads: the grid goes on along its z axis
+    n, dim = (1 << 28) + 3, 9
+    _print_case("preprocess_qk rows", n)
+    q = torch.zeros(1, 1, n, dim, dtype=torch.float16, device=DEV)
+    q.view(-1)[:: 4099] = 1.5
+    q[0, 0, -5:] = torch.arange(45, device=DEV).view(5, 9).to(torch.float16)
+    k = torch.ones(1, 1, 2, dim, dtype=torch.float16, device=DEV)
+    qo, ko = vcx.preprocess_qk(q, k, True, False)
+    for part, got in zip(q.chunk(16, dim=2), qo.chunk(16, dim=2)):
+        assert torch.equal(got, part.float())
+    assert torch.equal(ko, torch.zeros_like(ko))
+
+
 @pytest.mark.parametrize("dim,pad", [(64, 0), (64, 2), (128, 0), (128, 4), (128, 3), (96, 0)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
 @pytest.mark.parametrize("k_smooth,rotate", [(False, True), (True, False), (True, True)])
