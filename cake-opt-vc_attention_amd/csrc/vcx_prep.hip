@@ -480,18 +480,15 @@ __device__ inline void load_quad(const void* x, int64_t i, float (&v)[4]) {
   }
 }
 
-// Rows per thread of pre_rows_kernel: four, but one where entries move one by one and no mean is
-// subtracted. Four rows share a load of the mean; without one they only leave fewer waves to
-// hide the loads. fp16 [1,24,37741,37], rotated, one / four: 184 / 201 us without the mean, 233 /
-// 226 us with it.
-template <bool WIDE, bool MEAN>
-constexpr int kPreRows = WIDE || MEAN ? 4 : 1;
-
 // Blocks of pre_rows_kernel along the grid's x; more of them go on along z, as the threads along
 // one axis stay below 2^32.
 constexpr int64_t kRowsGridX = int64_t(1) << 22;
 
-// grid (tiles, B*H), D threads: binary64 sum of channel d over the tile's keys in key order.
+// grid (tiles, B*H), D threads: binary64 sum of channel d over the tile's keys in key order, the
+// loads of 16 keys in flight. One-wave blocks of four channels per thread, which move 8 or 16 bytes per
+// load, are no faster at any size (centring and rotation at [1,28,37741,128] bf16: 332 us with either)
+// and slower the fewer the tiles, as a lane's chain of additions is four times as long ([1,2,1000,64]
+// 13.9 us with these, 8.6 us so; [1,24,16001,64] 64.8 and 59.3 us).
 template <int DT>
 __global__ __launch_bounds__(128) void pre_tile_sum_kernel(const void* x, int64_t H, int64_t n, int64_t sb,
                                                            int64_t sh, int64_t sn, double* part) {
@@ -499,48 +496,18 @@ __global__ __launch_bounds__(128) void pre_tile_sum_kernel(const void* x, int64_
   const int d = threadIdx.x, D = blockDim.x;
   const int64_t off = (bh / H) * sb + (bh % H) * sh + d;
   const int64_t r0 = t * kTile, r1 = r0 + kTile < n ? r0 + kTile : n;
+  constexpr int kBatch = 16;
   double s = 0.0;
   int64_t r = r0;
-  for (; r + 8 <= r1; r += 8) {
-    float v[8];
+  for (; r + kBatch <= r1; r += kBatch) {
+    float v[kBatch];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) v[i] = elem<DT>(x, off + (r + i) * sn);
+    for (int i = 0; i < kBatch; ++i) v[i] = elem<DT>(x, off + (r + i) * sn);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) s = __dadd_rn(s, static_cast<double>(v[i]));
+    for (int i = 0; i < kBatch; ++i) s = __dadd_rn(s, static_cast<double>(v[i]));
   }
   for (; r < r1; ++r) s = __dadd_rn(s, static_cast<double>(elem<DT>(x, off + r * sn)));
   part[(bh * tiles + t) * D + d] = s;
-}
-
-// The same sums where every row starts on 8 bytes and D is 64 or 128: grid (ceil(tiles *
-// LT / 64), B*H) one-wave blocks, LT = D / 4 lanes per tile with four adjacent channels each.
-// One 8-byte load (16 for binary32) brings a lane four channels of a key and kBatch keys are
-// in flight, where a thread per channel moves 2 bytes per load ([1,28,37741,128] bf16:
-// 79 us with that, 46 us with this).
-template <int DT, int D>
-__global__ __launch_bounds__(64) void pre_tile_sum_wide_kernel(const void* x, int64_t H, int64_t n, int64_t sb,
-                                                               int64_t sh, int64_t sn, int64_t tiles, double* part) {
-  constexpr int LT = D / 4, kBatch = 16;
-  const int64_t bh = blockIdx.y, t = static_cast<int64_t>(blockIdx.x) * (64 / LT) + threadIdx.x / LT;
-  const int c = threadIdx.x % LT;
-  if (t >= tiles) return;
-  const int64_t off = (bh / H) * sb + (bh % H) * sh + 4 * c;
-  const int64_t r0 = t * kTile, r1 = r0 + kTile < n ? r0 + kTile : n;
-  double s[4] = {0.0, 0.0, 0.0, 0.0};
-  for (int64_t r = r0; r < r1; r += kBatch) {
-    float v[kBatch][4];
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i) load_quad<DT>(x, off + (r + i < r1 ? r + i : r) * sn, v[i]);
-#pragma unroll
-    for (int i = 0; i < kBatch; ++i)
-      if (r + i < r1) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[j] = __dadd_rn(s[j], static_cast<double>(v[i][j]));
-      }
-  }
-  double2* dst = reinterpret_cast<double2*>(part + (bh * tiles + t) * D + 4 * c);
-  dst[0] = make_double2(s[0], s[1]);
-  dst[1] = make_double2(s[2], s[3]);
 }
 
 // grid (ceil(n / RPB) (+ 1 with KM), B*H): out = x - mean (mean nullable), rotated with ROT,
@@ -551,8 +518,9 @@ __global__ __launch_bounds__(64) void pre_tile_sum_wide_kernel(const void* x, in
 // byte loads, 16-byte stores), without it one by one. The kernel streams: at [1,28,37741,128]
 // bf16 one row and one-entry loads per thread took 230 us for Q and 442 us with the mean, this
 // form 148 and 139 us (5.8 TB/s).
-// Input rows and outputs are touched once here, non-temporally, so that K stays in the
-// memory-side cache between its sums and this pass.
+// Outputs in 16-byte pieces go past the caches (non-temporal), so that K stays in the memory-side
+// cache between its sums and this pass. One by one without rotation, adjacent lanes take adjacent
+// entries ([1,24,37741,72] bf16: 382 us with four adjacent entries per lane, 198 us so).
 // KM (Q's launch): blocks (0, bh) form head bh's K mean instead, beside the Q rows.
 template <int DT, int W, bool ROT, bool WIDE, bool KM, int NR>
 __global__ __launch_bounds__(kThreads) void pre_rows_kernel(const void* x, int64_t H, int64_t n, int D, int64_t sb,
@@ -571,7 +539,7 @@ __global__ __launch_bounds__(kThreads) void pre_rows_kernel(const void* x, int64
   const int tid = threadIdx.x, c = tid % L;
   const int64_t bh = blockIdx.y, r0 = blk * RPB + tid / L;
   const int64_t head = (bh / H) * sb + (bh % H) * sh;
-  auto channel = [&](int j) { return SPLIT ? 4 * c + (j & 3) + 64 * (j >> 2) : c * CPT + j; };
+  auto channel = [&](int j) { return !ROT && !WIDE ? c + L * j : SPLIT ? 4 * c + (j & 3) + 64 * (j >> 2) : c * CPT + j; };
   float v[NR][CPT];
 #pragma unroll
   for (int i = 0; i < NR; ++i) {
@@ -1255,16 +1223,11 @@ int preprocess_launch(const void* q, const void* k, int64_t BH, int64_t H, int64
     return (D == 64 || D == 128) && aligned(x, kQuad) && sb % 4 == 0 && sh % 4 == 0 && sn % 4 == 0;
   };
   const bool q_wide = quads(q, q_sb, q_sh, q_sn) && aligned(q_out, 16);
-  const bool k_rows = quads(k, k_sb, k_sh, k_sn), k_wide = k_rows && aligned(k_out, 16);
+  const bool k_wide = quads(k, k_sb, k_sh, k_sn) && aligned(k_out, 16);
   KMeanArgs kma{};
   if (k_smooth) {
     kma = KMeanArgs{part, tiles, Nk, mean, nullptr};
-    if (k_rows && D == 128)
-      pre_tile_sum_wide_kernel<DT, 128><<<dim3(cdiv(tiles, 2), BH), 64, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, tiles, part);
-    else if (k_rows)
-      pre_tile_sum_wide_kernel<DT, 64><<<dim3(cdiv(tiles, 4), BH), 64, 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, tiles, part);
-    else
-      pre_tile_sum_kernel<DT><<<dim3(tiles, BH), static_cast<unsigned>(D), 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, part);
+    pre_tile_sum_kernel<DT><<<dim3(tiles, BH), static_cast<unsigned>(D), 0, st>>>(k, H, Nk, k_sb, k_sh, k_sn, part);
     VCX_LAUNCHED("pre_tile_sum_kernel");
   }
   int W = 1;
@@ -1284,12 +1247,25 @@ int preprocess_launch(const void* q, const void* k, int64_t BH, int64_t H, int64
              0, st>>>(x, H, n, static_cast<int>(D), sb, sh, sn, mu, out, norm, kma);
     };
     const float* none = nullptr;
-    auto launch = [&](bool wide, auto km, auto centre, auto... args) {
+    auto launch = [&](bool wide, auto km, auto centre, const void* x, int64_t n, auto... args) {
       constexpr bool MEAN = decltype(centre)::value;
+      auto nr = [&](auto w) {
+        constexpr bool WIDE = decltype(w)::value;
+        // Four rows per thread share a load of the mean and leave more loads in flight, one row more
+        // waves: four from about two blocks of them per CU on, and one wherever entries move one
+        // by one and four would gain nothing (no mean, or a plain difference of wide rows). Q and K,
+        // whole call in us, one row / four rows: [1,2,1000,128] rotated 4.6 / 6.8, [1,8,4000,128] centred and
+        // rotated 23.6 / 21.7, [1,28,37741,16] centred 99.9 / 80.9, [1,28,37741,72] centred 298 / 323.
+        if constexpr (WIDE || (MEAN && (ROT || WW <= 32))) {
+          if (BH * cdiv(n, 4 * kThreads / L) >= (WIDE && MEAN ? 256 : 512))
+            return rows(w, km, std::integral_constant<int, 4>(), x, n, args...);
+        }
+        rows(w, km, std::integral_constant<int, 1>(), x, n, args...);
+      };
       if constexpr (WW == 64 || WW == 128) {
-        if (wide) return rows(std::true_type(), km, std::integral_constant<int, kPreRows<true, MEAN>>(), args...);
+        if (wide) return nr(std::true_type());
       }
-      rows(std::false_type(), km, std::integral_constant<int, kPreRows<false, MEAN>>(), args...);
+      nr(std::false_type());
     };
     if (k_smooth) launch(q_wide, std::true_type(), std::false_type(), q, Nq, q_sb, q_sh, q_sn, none, q_out);
     else launch(q_wide, std::false_type(), std::false_type(), q, Nq, q_sb, q_sh, q_sn, none, q_out);

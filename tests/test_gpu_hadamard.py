@@ -107,6 +107,23 @@ def test_preprocess_qk_bit_exact_and_matrix_oracle(dim, dtype, k_smooth, rotate)
     torch.testing.assert_close(kd.cpu(), k, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("dim", [128, 64, 100, 24, 9])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("k_smooth,rotate", [(False, False), (False, True), (True, False), (True, True)])
+def test_preprocess_qk_one_and_four_rows_per_thread(dim, dtype, k_smooth, rotate):
+    # Q's 2000 rows of eight heads take one row per thread, K's 4097 four where that pays (512 blocks of
+    # 64 rows; centred rows of 64 and 128 from 256 on), with a ragged last block either way.
+    _print_case("preprocess_qk rows per thread", dim, dtype, k_smooth, rotate)
+    gen = torch.Generator().manual_seed(23)
+    name = {torch.float32: "float32", torch.bfloat16: "bfloat16"}[dtype]
+    arg = (lambda x: x.numpy()) if dtype == torch.float32 else bits
+    q, k = [torch.randn(1, 8, n, dim, generator=gen).to(dtype) for n in (2000, 4097)]
+    qo, ko = vcx.preprocess_qk(q.to(DEV), k.to(DEV), k_smooth, rotate)
+    eq, ek = o.preprocess_qk(arg(q), arg(k), k_smooth=k_smooth, hadamard=rotate, dtype=name)
+    np.testing.assert_array_equal(qo.cpu().numpy(), eq)
+    np.testing.assert_array_equal(ko.cpu().numpy(), ek)
+
+
 def test_preprocess_qk_more_rows_than_one_grid_axis_holds():
     # 2^28 + 3 rows in blocks of 16 are more than 2^32 threads: the grid goes on along its z axis
     n, dim = (1 << 28) + 3, 9
