@@ -64,6 +64,23 @@ def cosine(a, b):
     return float(a @ b / max(np.linalg.norm(a) * np.linalg.norm(b), 1e-300))
 
 
+def both_ways(forward, payload, *args, p_rows, **options):
+    """(out, P bytes) of a fused call on the payload (q, k, v, qs, ks, vs[, means]) as given, which a
+    call of few rows runs as split pieces, and on as many copies of it as the streaming blocks need
+    to be chosen (more 64-row pieces than CUs). The copies' results are equal, so one of them is
+    returned, as is one run without a P dump."""
+    B, H, nq = payload[0].shape[:3]
+    cus = torch.cuda.get_device_properties(payload[0].device).multi_processor_count
+    for n in (1, cus // (B * H * (-(-nq // 64))) + 1):
+        many = [None if x is None else x.repeat(n, *(1,) * (x.dim() - 1)) for x in payload]
+        out, codes = forward(*many, *args, p_rows=p_rows, **options)
+        plain = forward(*many, *args, **options)
+        assert torch.equal(plain, out)
+        for x in (out, codes):
+            assert torch.equal(x, x[:B].repeat(n, 1, 1, 1))
+        yield out[:B], codes[:B]
+
+
 def output_bound(actual, expected):
     """Elementwise tolerance of the bf16/fp16 output vs the fp32-simulated oracle.
 

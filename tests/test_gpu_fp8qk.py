@@ -81,7 +81,7 @@ def test_prepare_qk_fp8_strided_nhd():
 
 # ------------------------------------------------------------------ fused FP8 forward
 
-from helpers import cosine, logical_to_storage, make_qkv, output_bound, storage_to_logical  # noqa: E402
+from helpers import both_ways, cosine, logical_to_storage, make_qkv, output_bound, storage_to_logical  # noqa: E402
 
 MODES = {"folded": (True, True), "unfused": (True, False), "control": (False, False)}  # expcast, affine
 
@@ -90,11 +90,13 @@ def _to_dev(a):
     return torch.from_numpy(np.ascontiguousarray(a)).to(DEV)
 
 
+def _payload(st):
+    v8 = _to_dev(logical_to_storage(st["v"], vcx.value_token()))
+    return _to_dev(st["q"]), _to_dev(st["k"]), v8, _to_dev(st["qs"]), _to_dev(st["ks"]), _to_dev(st["vs"])
+
+
 def _run(st, expcast, affine, rows):
-    tok = vcx.value_token()
-    v8 = _to_dev(logical_to_storage(st["v"], tok))
-    return vcx.forward_fp8(_to_dev(st["q"]), _to_dev(st["k"]), v8, _to_dev(st["qs"]), _to_dev(st["ks"]),
-                           _to_dev(st["vs"]), expcast, st["output_type"], st["scale"], affine=affine, p_rows=rows)
+    return vcx.forward_fp8(*_payload(st), expcast, st["output_type"], st["scale"], affine=affine, p_rows=rows)
 
 
 def _integer_state(B, H, Nq, Nk, D, seed, dtype="bfloat16"):
@@ -134,13 +136,14 @@ def test_fp8_forward_exact_scores_p_bytes_bit_exact(case, mode):
     _print_case("fp8 forward integer codes", case, mode)
     st = _integer_state(B, H, Nq, Nk, D, seed=Nq * 7 + Nk)
     st["expcast"] = expcast
-    out, pd = _run(st, expcast, affine, (0, Nq))
     eout, ecodes = o.reference(st, return_codes=True, affine=affine)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
+    for out, pd in both_ways(vcx.forward_fp8, _payload(st), expcast, st["output_type"], st["scale"], affine=affine,
+                             p_rows=(0, Nq)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 FWD_CASES = [  # B, H, Nq, Nk, D, dtype
@@ -197,22 +200,23 @@ def test_fp8_forward_gaussian_p_bytes_and_output(case, mode):
     _print_case("fp8 forward gaussian", case, mode)
     q, k, v = make_qkv(B, H, Nq, Nk, D, dt, seed=27)
     st = o.prepare_fp8(bits(q), bits(k), bits(v), expcast=expcast, dtype=dtype_name(dt))
-    out, pd = _run(st, expcast, affine, (0, Nq))
     eout, ecodes = o.reference(st, return_codes=True, affine=affine)
-    got_codes = pd.cpu().numpy()
-    # ExpCast codes, and E4M3 codes of nonnegative probabilities, are monotone in the byte
-    diff = np.abs(got_codes.astype(np.int32) - ecodes.astype(np.int32))
-    frac = float((diff != 0).mean())
-    print("P byte mismatches:", int((diff != 0).sum()), "of", diff.size, "max", int(diff.max()), flush=True)
-    assert diff.max() <= 1
-    assert frac <= 5e-4
-    got = out.float().cpu().numpy()
-    assert np.isfinite(got).all()
-    # the kernel's output is the attention its own P bytes define ...
-    err, bound = output_bound(got, _expected_from_codes(st, got_codes, expcast))
-    assert np.all(err <= bound), float((err - bound).max())
-    # ... and the rare one-code moves leave it next to the oracle's
-    assert cosine(got, eout) >= 0.9999
+    for out, pd in both_ways(vcx.forward_fp8, _payload(st), expcast, st["output_type"], st["scale"], affine=affine,
+                             p_rows=(0, Nq)):
+        got_codes = pd.cpu().numpy()
+        # ExpCast codes, and E4M3 codes of nonnegative probabilities, are monotone in the byte
+        diff = np.abs(got_codes.astype(np.int32) - ecodes.astype(np.int32))
+        frac = float((diff != 0).mean())
+        print("P byte mismatches:", int((diff != 0).sum()), "of", diff.size, "max", int(diff.max()), flush=True)
+        assert diff.max() <= 1
+        assert frac <= 5e-4
+        got = out.float().cpu().numpy()
+        assert np.isfinite(got).all()
+        # the kernel's output is the attention its own P bytes define ...
+        err, bound = output_bound(got, _expected_from_codes(st, got_codes, expcast))
+        assert np.all(err <= bound), float((err - bound).max())
+        # ... and the rare one-code moves leave it next to the oracle's
+        assert cosine(got, eout) >= 0.9999
 
 
 @pytest.mark.parametrize("cast", [False, True])

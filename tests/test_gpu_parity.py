@@ -11,8 +11,8 @@ import pytest
 import torch
 
 import vcx
-from helpers import (FOLD_CODE_FOLDED, FOLD_CODE_UNFUSED, bits, cosine, dtype_name, folded_encode_payload,
-                     logical_to_storage, make_qkv, output_bound, storage_to_logical)
+from helpers import (FOLD_CODE_FOLDED, FOLD_CODE_UNFUSED, bits, both_ways, cosine, dtype_name,
+                     folded_encode_payload, logical_to_storage, make_qkv, output_bound, storage_to_logical)
 from oracle import vc_oracle as o
 
 pytestmark = pytest.mark.gpu
@@ -466,20 +466,15 @@ def test_attention_p_bytes_bit_exact_and_output_tolerance(case):
     to = _to_dev
     v8 = to(logical_to_storage(st["v"], tok)).view(torch.float8_e4m3fn)
     means = to(st["means"]).view(torch.float16) if smooth else None
-    rows = (0, Nq)
-    out, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), means,
-                          True, smooth, st["output_type"], st["scale"], p_rows=rows)
     eout, ecodes = o.reference(st, return_codes=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    assert np.isfinite(got).all()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
-    # the production (non-dump) kernel gives the same output bits
-    out2 = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), means,
-                       True, smooth, st["output_type"], st["scale"])
-    assert torch.equal(out2, out)
+    for out, pd in both_ways(vcx.forward, (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), means),
+                             True, smooth, st["output_type"], st["scale"], p_rows=(0, Nq)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        assert np.isfinite(got).all()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 def test_uniform_attention_three_unequal_blocks_known_answer():
@@ -606,12 +601,12 @@ def test_last_tile_rounding_order_known_answer_on_gpu(nk):
     st = rounding_order_payload(nk)
     to = _to_dev
     v8 = to(st["v"]).view(torch.float8_e4m3fn)
-    _, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None,
-                        True, False, 1, st["scale"], p_rows=(0, 1))
-    codes = pd.cpu().numpy()
-    assert codes[0, 0, 0, 0] == 120
-    assert codes[0, 0, 0, 1] == (ORDER_CODE_LAST if nk <= 128 else ORDER_CODE_OTHER)
-    assert np.all(codes[0, 0, 0, 2:] == 0)
+    for _, pd in both_ways(vcx.forward, (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None),
+                           True, False, 1, st["scale"], p_rows=(0, 1)):
+        codes = pd.cpu().numpy()
+        assert codes[0, 0, 0, 0] == 120
+        assert codes[0, 0, 0, 1] == (ORDER_CODE_LAST if nk <= 128 else ORDER_CODE_OTHER)
+        assert np.all(codes[0, 0, 0, 2:] == 0)
 
 
 FULL = [  # name, B, H, N, D, kind: the BASELINE smoothing configurations in full
@@ -658,11 +653,12 @@ BLOCK = [  # B, H, Nq, Nk, D, dtype
     (1, 2, 300, 700, 128, torch.bfloat16),
     (2, 1, 129, 257, 64, torch.float16),
     (1, 1, 1, 1, 128, torch.bfloat16),
-    # the deferred mean term: 36 tiles (two full 16-tile chunks, the 17-slot ring wraps
-    # twice), a chunk that ends on the last tile, and a last tile that opens a chunk
+    # the deferred mean term: 36 tiles (two full 16-tile chunks, the streaming blocks' 17-slot
+    # ring wraps twice), chunks that end on the last tile, and a last tile that opens a chunk
     (1, 1, 64, 4500, 128, torch.bfloat16),
     (1, 2, 40, 2048, 64, torch.float16),
     (1, 1, 33, 2049, 128, torch.bfloat16),
+    (1, 1, 17, 6144, 64, torch.bfloat16),
 ]
 
 
@@ -678,16 +674,16 @@ def test_attention_block_scales_p_bytes_and_output(case):
     tok = vcx.value_token()
     to = _to_dev
     v8 = to(logical_to_storage(st["v"], tok)).view(torch.float8_e4m3fn)
-    out, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]),
-                          to(st["means"]).view(torch.float16), True, True, st["output_type"], st["scale"],
-                          channel_scale=False, p_rows=(0, Nq))
     eout, ecodes = o.reference(st, return_codes=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    assert np.isfinite(got).all()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
+    payload = (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), to(st["means"]).view(torch.float16))
+    for out, pd in both_ways(vcx.forward, payload, True, True, st["output_type"], st["scale"], channel_scale=False,
+                             p_rows=(0, Nq)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        assert np.isfinite(got).all()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 def test_sageattn_vc_block_scale_end_to_end():
@@ -748,6 +744,10 @@ CONTROL = [  # B, H, Nq, Nk, D, dtype, V mode
     (1, 1, 129, 513, 64, torch.bfloat16, "channel"),
     (1, 2, 257, 385, 128, torch.float16, "channel"),
     (1, 2, 300, 700, 128, torch.bfloat16, "block"),
+    # the deferred mean term over more than two chunks of 16 tiles
+    (1, 1, 33, 4500, 128, torch.bfloat16, "channel"),
+    (1, 1, 20, 4500, 64, torch.float16, "channel"),
+    (1, 1, 20, 6144, 64, torch.bfloat16, "block"),
 ]
 
 
@@ -766,19 +766,16 @@ def test_control_path_p_bytes_and_output(case):
     to = _to_dev
     v8 = to(logical_to_storage(st["v"], vcx.value_token())).view(torch.float8_e4m3fn)
     means = to(st["means"]).view(torch.float16) if smooth else None
-    out, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), means,
-                          False, smooth, st["output_type"], st["scale"], channel_scale=vmode != "block",
-                          p_rows=(0, Nq))
     eout, ecodes = o.reference(st, return_codes=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    assert np.isfinite(got).all()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
-    out2 = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), means,
-                       False, smooth, st["output_type"], st["scale"], channel_scale=vmode != "block")
-    assert torch.equal(out2, out)
+    for out, pd in both_ways(vcx.forward, (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), means),
+                             False, smooth, st["output_type"], st["scale"], channel_scale=vmode != "block",
+                             p_rows=(0, Nq)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        assert np.isfinite(got).all()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 @pytest.mark.parametrize("dim", [64, 128])
@@ -792,15 +789,15 @@ def test_control_path_far_logits_p_bytes_and_output(dim):
     st = o.prepare(bits(q), bits(k), bits(v), expcast=False, v_smooth=False, dtype="bfloat16")
     to = _to_dev
     v8 = to(logical_to_storage(st["v"], vcx.value_token())).view(torch.float8_e4m3fn)
-    out, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None,
-                          False, False, st["output_type"], st["scale"], p_rows=(0, 200))
     eout, ecodes = o.reference(st, return_codes=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
     assert (ecodes == 0).mean() > 0.5  # most probabilities round to byte 0
-    got = out.float().cpu().numpy()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
+    for out, pd in both_ways(vcx.forward, (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None),
+                             False, False, st["output_type"], st["scale"], p_rows=(0, 200)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 @pytest.mark.parametrize("dim,nk", [(64, 130), (64, 640), (64, 700), (128, 256), (128, 513), (128, 768)])
@@ -912,17 +909,14 @@ def test_folded_encode_p_bytes_bit_exact_and_output(case):
     st = _oracle_state(q, k, v, False, dt)
     to = _to_dev
     v8 = to(logical_to_storage(st["v"], vcx.value_token())).view(torch.float8_e4m3fn)
-    out, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None,
-                          True, False, st["output_type"], st["scale"], affine=True, p_rows=(0, Nq))
     eout, ecodes = o.reference(st, return_codes=True, affine=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
-    out2 = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None,
-                       True, False, st["output_type"], st["scale"], affine=True)
-    assert torch.equal(out2, out)
+    for out, pd in both_ways(vcx.forward, (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None),
+                             True, False, st["output_type"], st["scale"], affine=True, p_rows=(0, Nq)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 @pytest.mark.parametrize("extreme, code", [((), FOLD_CODE_FOLDED), ((3,), FOLD_CODE_UNFUSED), ((19,), FOLD_CODE_FOLDED)])
@@ -934,18 +928,18 @@ def test_folded_encode_known_answer_and_group_fallback_on_gpu(extreme, code):
     _print_case("folded encode KA", extreme)
     to = _to_dev
     v8 = to(logical_to_storage(s["v"], vcx.value_token())).view(torch.float8_e4m3fn)
-    _, pd = vcx.forward(to(s["q"]), to(s["k"]), v8, to(s["qs"]), to(s["ks"]), to(s["vs"]), None,
-                        True, False, 1, s["scale"], affine=True, p_rows=(0, 32))
-    got = pd.cpu().numpy()
-    assert got[0, 0, 0, 96] == code and got[0, 0, 0, 45] == 120
     _, ecodes = o.reference(s, return_codes=True, affine=True)
-    np.testing.assert_array_equal(got, ecodes)
+    for _, pd in both_ways(vcx.forward, (to(s["q"]), to(s["k"]), v8, to(s["qs"]), to(s["ks"]), to(s["vs"]), None),
+                           True, False, 1, s["scale"], affine=True, p_rows=(0, 32)):
+        got = pd.cpu().numpy()
+        assert got[0, 0, 0, 96] == code and got[0, 0, 0, 45] == 120
+        np.testing.assert_array_equal(got, ecodes)
 
 
 @pytest.mark.parametrize("factor", [1e4, 1e-36], ids=["large", "tiny"])
 def test_folded_encode_known_answer_when_the_head_precheck_fails(factor):
-    # The kernel first tests the fold conditions for a whole head at once (the extreme K
-    # scales, a |logit| bound per row). Scaling the last tile's K scales by 1e4 (the bound
+    # The streaming blocks first test the fold conditions for a whole head at once (the extreme
+    # K scales, a |logit| bound per row); pieces test them tile by tile. Scaling the last tile's K scales by 1e4 (the bound
     # passes 128) or 1e-36 (the smallest scale is subnormal) fails that test, so tile 0
     # tests the conditions itself: they hold there, and key 96 keeps its folded byte.
     s = folded_encode_payload()
@@ -954,19 +948,19 @@ def test_folded_encode_known_answer_when_the_head_precheck_fails(factor):
     _print_case("folded encode KA, head precheck fails", factor)
     to = _to_dev
     v8 = to(logical_to_storage(s["v"], vcx.value_token())).view(torch.float8_e4m3fn)
-    _, pd = vcx.forward(to(s["q"]), to(s["k"]), v8, to(s["qs"]), to(s["ks"]), to(s["vs"]), None,
-                        True, False, 1, s["scale"], affine=True, p_rows=(0, 32))
-    got = pd.cpu().numpy()
-    assert got[0, 0, 0, 96] == FOLD_CODE_FOLDED and got[0, 0, 0, 45] == 120
     _, ecodes = o.reference(s, return_codes=True, affine=True)
-    np.testing.assert_array_equal(got, ecodes)
+    for _, pd in both_ways(vcx.forward, (to(s["q"]), to(s["k"]), v8, to(s["qs"]), to(s["ks"]), to(s["vs"]), None),
+                           True, False, 1, s["scale"], affine=True, p_rows=(0, 32)):
+        got = pd.cpu().numpy()
+        assert got[0, 0, 0, 96] == FOLD_CODE_FOLDED and got[0, 0, 0, 45] == 120
+        np.testing.assert_array_equal(got, ecodes)
 
 
 @pytest.mark.parametrize("dim", [64, 128])
 @pytest.mark.parametrize("factor", [10.0, 300.0, 1e-36], ids=["moderate", "large", "tiny"])
 def test_folded_encode_per_tile_conditions_with_k_scale_outliers(dim, factor):
-    # The K scales of tile 2 (of 8) multiplied by `factor`: the head-wide test of the fold
-    # conditions fails, and every tile tests them itself. moderate: every |m'| stays <= 128
+    # The K scales of tile 2 (of 8) multiplied by `factor`: the streaming blocks' head-wide test of
+    # the fold conditions fails, and every tile tests them itself (as in pieces always). moderate: every |m'| stays <= 128
     # (all tiles fold); large: tile 2's logits pass 128, so from tile 2 on every row group
     # takes the unfused bytes; tiny: tile 2's scale is subnormal (tile 2 unfused only).
     # P bytes exact against the oracle, output within the bound.
@@ -977,13 +971,13 @@ def test_folded_encode_per_tile_conditions_with_k_scale_outliers(dim, factor):
     _print_case("fold conditions per tile", dim, factor)
     to = _to_dev
     v8 = to(logical_to_storage(st["v"], vcx.value_token())).view(torch.float8_e4m3fn)
-    out, pd = vcx.forward(to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None,
-                          True, False, st["output_type"], st["scale"], affine=True, p_rows=(0, 160))
     eout, ecodes = o.reference(st, return_codes=True, affine=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
+    for out, pd in both_ways(vcx.forward, (to(st["q"]), to(st["k"]), v8, to(st["qs"]), to(st["ks"]), to(st["vs"]), None),
+                             True, False, st["output_type"], st["scale"], affine=True, p_rows=(0, 160)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
 
 
 def test_deferred_mean_restore_rising_maximum_across_chunks():
@@ -1004,15 +998,15 @@ def test_deferred_mean_restore_rising_maximum_across_chunks():
     st = _oracle_state(q, k, v, True, torch.bfloat16)
     tok = vcx.value_token()
     v8 = _to_dev(logical_to_storage(st["v"], tok)).view(torch.float8_e4m3fn)
-    out, pd = vcx.forward(_to_dev(st["q"]), _to_dev(st["k"]), v8, _to_dev(st["qs"]), _to_dev(st["ks"]),
-                          _to_dev(st["vs"]), _to_dev(st["means"]).view(torch.float16), True, True,
-                          st["output_type"], st["scale"], p_rows=(0, 160))
     eout, ecodes = o.reference(st, return_codes=True)
-    np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
-    got = out.float().cpu().numpy()
-    err, bound = output_bound(got, eout)
-    assert np.all(err <= bound), float((err - bound).max())
-    assert cosine(got, eout) >= 0.9999
+    payload = (_to_dev(st["q"]), _to_dev(st["k"]), v8, _to_dev(st["qs"]), _to_dev(st["ks"]), _to_dev(st["vs"]),
+               _to_dev(st["means"]).view(torch.float16))
+    for out, pd in both_ways(vcx.forward, payload, True, True, st["output_type"], st["scale"], p_rows=(0, 160)):
+        np.testing.assert_array_equal(pd.cpu().numpy(), ecodes)
+        got = out.float().cpu().numpy()
+        err, bound = output_bound(got, eout)
+        assert np.all(err <= bound), float((err - bound).max())
+        assert cosine(got, eout) >= 0.9999
 
 
 @pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
