@@ -44,8 +44,8 @@
 // PM = 0 is the Sage FP8 control path (expcast=False; vc_sm90.cu:177,
 // attn_utils.cuh:355-455): a.sm = RN(sm * RN(log2 e)), base/factor as above,
 // m' = max(m, max fmaf(base, factor, -8.807)), P = E4M3(exp2(fmaf(base, factor, -m'))) with
-// the correctly rounded binary32 exp2 (fp8_exp2_word: v_exp_f32, rechecked in binary64 next
-// to an E4M3 rounding midpoint, which fp8_exp2_gap looks for); den and the mean restore use the unrounded sum of P.
+// the correctly rounded binary32 exp2 (fp8_exp2_quick: v_exp_f32, and next to an E4M3 rounding
+// midpoint, which fp8_exp2_gap looks for, fp8_exp2_word: rechecked in binary64); den and the mean restore use the unrounded sum of P.
 #include "vcx_attn.hpp"
 
 #include <functional>
@@ -503,9 +503,10 @@ extern "C" int vcx_attention_fwd_fp8(const uint8_t* q8, const uint8_t* k8, const
 
 namespace vcx {
 namespace {
-// One thread per four inputs: the control path's probability bytes via fp8_exp2_word
-// (SAT: the saturating lower neighbours the fused kernel uses; else the 64-bit pair form).
-template <bool SAT>
+// One thread per four inputs: the control path's probability bytes as Wave::bytes forms them
+// (LIFT: in the general copy of the tile loop and in pieces; else in the copy with the cheap
+// midpoint test).
+template <bool LIFT>
 __global__ void fp8_exp2_probe_kernel(const float* x, uint8_t* y, int64_t n) {
   const int64_t i = (static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
   if (i >= n) return;
@@ -515,7 +516,8 @@ __global__ void fp8_exp2_probe_kernel(const float* x, uint8_t* y, int64_t n) {
     xs[r] = i + r < n ? x[i + r] : -INFINITY;
     pr[r] = __builtin_amdgcn_exp2f(xs[r]);
   }
-  const uint32_t w = fp8_exp2_word<SAT>(xs, pr);
+  uint32_t gap = 0xffffffffu, w = fp8_exp2_quick<LIFT>(pr, gap);
+  if (gap <= kFp8Gap) w = fp8_exp2_word(xs, pr);
 #pragma unroll
   for (int r = 0; r < 4; ++r)
     if (i + r < n) y[i + r] = static_cast<uint8_t>(w >> (8 * r));

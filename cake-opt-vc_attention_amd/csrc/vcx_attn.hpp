@@ -595,13 +595,8 @@ struct Wave {
 #pragma unroll
           for (int r = 0; r < 4; ++r) pr[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(bs[j][r], f, -mx));
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const uint32_t g = fp8_exp2_gap<!PRE>(pr[r]);
-            gap = gap < g ? gap : g;
-            ls += pr[r];
-          }
-          const int w = __builtin_amdgcn_cvt_pk_fp8_f32(pr[0], pr[1], 0, false);
-          Pq[j] = __builtin_amdgcn_cvt_pk_fp8_f32(pr[2], pr[3], w, true);
+          for (int r = 0; r < 4; ++r) ls += pr[r];
+          Pq[j] = static_cast<int>(fp8_exp2_quick<!PRE>(pr, gap));
         }
         if (__builtin_expect(gap <= kFp8Gap, 0)) {
           ls = ls0;
@@ -617,7 +612,7 @@ struct Wave {
               pr[r] = __builtin_amdgcn_exp2f(xs[r]);
               low = fminf(low, pr[r]);
             }
-            Pq[j] = static_cast<int>(fp8_exp2_word<true>(xs, pr));
+            Pq[j] = static_cast<int>(fp8_exp2_word(xs, pr));
 #pragma unroll
             for (int r = 0; r < 4; ++r) ls += pr[r];
           }

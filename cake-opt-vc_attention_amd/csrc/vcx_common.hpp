@@ -108,12 +108,8 @@ __device__ inline uint32_t e4m3_sat(float x) {
 // input). The bytes of p - 2 ulps and p + 2 ulps agree unless an E4M3 rounding midpoint lies
 // within two ulps of p; only then does the lane recompute exp2 in binary64 and round it once
 // to binary32 (p is updated to that value). The upper neighbours of two probabilities come
-// from one 64-bit add (v_lshl_add_u64). SAT = true (what the fused kernel's recheck uses) forms the
-// lower neighbours with a saturating subtraction per probability. SAT = false uses one 64-bit
-// subtraction per pair, half the instructions, but a borrow out of a low half below 2 ulps (p
-// = 0 or the smallest subnormal, i.e. x below about -149) then yields a NaN byte and a
-// needless recheck: bytes stay right, but rows whose scores lie more than about 103 nats
-// below the row maximum recheck on most tiles. The fused kernel asks fp8_exp2_gap first.
+// from one 64-bit add (v_lshl_add_u64), the lower ones from a saturating subtraction each. The
+// fused kernel asks fp8_exp2_quick first.
 // Reference: the probability byte of sal/sageattention_local/vc_reference.py:68-75 and
 // sal/csrc/qattn/attn_utils.cuh:355-455.
 // fp8_exp2_bounds gives the bytes of both neighbour sets (lo, hi); fp8_exp2_word resolves a
@@ -121,7 +117,6 @@ __device__ inline uint32_t e4m3_sat(float x) {
 // recheck.
 __device__ __noinline__ inline float exp2_via_f64(float x) { return static_cast<float>(exp2(static_cast<double>(x))); }
 
-template <bool SAT>
 __device__ inline void fp8_exp2_bounds(const float (&p)[4], uint32_t& lo, uint32_t& hi) {
   constexpr uint64_t kTwoUlps = 0x0000000200000002ull;
   float dn[4], up[4];
@@ -131,15 +126,9 @@ __device__ inline void fp8_exp2_bounds(const float (&p)[4], uint32_t& lo, uint32
     const uint64_t u = pr + kTwoUlps;
     up[2 * h] = __uint_as_float(static_cast<uint32_t>(u));
     up[2 * h + 1] = __uint_as_float(static_cast<uint32_t>(u >> 32));
-    if constexpr (SAT) {
 #pragma unroll
-      for (int r = 2 * h; r < 2 * h + 2; ++r)
-        dn[r] = __uint_as_float(__builtin_elementwise_sub_sat(__float_as_uint(p[r]), 2u));  // p >= 0: stops at +0
-    } else {
-      const uint64_t d = pr - kTwoUlps;
-      dn[2 * h] = __uint_as_float(static_cast<uint32_t>(d));
-      dn[2 * h + 1] = __uint_as_float(static_cast<uint32_t>(d >> 32));
-    }
+    for (int r = 2 * h; r < 2 * h + 2; ++r)
+      dn[r] = __uint_as_float(__builtin_elementwise_sub_sat(__float_as_uint(p[r]), 2u));  // p >= 0: stops at +0
   }
   lo = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(dn[0], dn[1], 0, false));
   lo = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(dn[2], dn[3], static_cast<int>(lo), true));
@@ -149,10 +138,9 @@ __device__ inline void fp8_exp2_bounds(const float (&p)[4], uint32_t& lo, uint32
 
 // The four bytes themselves: the lower neighbours' bytes when both neighbours agree, else the
 // binary64 recheck.
-template <bool SAT = false>
 __device__ inline uint32_t fp8_exp2_word(const float (&x)[4], float (&p)[4]) {
   uint32_t lo, hi;
-  fp8_exp2_bounds<SAT>(p, lo, hi);
+  fp8_exp2_bounds(p, lo, hi);
   if (__builtin_expect(lo != hi, 0)) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) p[r] = exp2_via_f64(x[r]);
@@ -175,6 +163,17 @@ __device__ inline uint32_t fp8_exp2_gap(float p) {
   uint32_t u = __float_as_uint(p);
   if constexpr (LIFT) u = u > kLift ? u : kLift;
   return (u << 13) + (2u << 13);
+}
+// Four probabilities' own bytes; gap keeps the smallest fp8_exp2_gap seen.
+template <bool LIFT>
+__device__ __forceinline__ uint32_t fp8_exp2_quick(const float (&p)[4], uint32_t& gap) {
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const uint32_t g = fp8_exp2_gap<LIFT>(p[r]);
+    gap = gap < g ? gap : g;
+  }
+  const int w = __builtin_amdgcn_cvt_pk_fp8_f32(p[0], p[1], 0, false);
+  return static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(p[2], p[3], w, true));
 }
 
 // ExpCast constants (exact fp32 values of the reference, expcast.cuh:7).

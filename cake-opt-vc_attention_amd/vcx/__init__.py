@@ -543,8 +543,9 @@ def expcast_codes(x):
 @_device_call
 def fp8_exp2_codes(x, last_tile: bool = False):
     """E4M3 bytes of the control path's probabilities exp2(x), from the fused kernel's device
-    code (last_tile: the saturating window form, which the kernel runs on every tile; else
-    the 64-bit pair form; the bytes are the same)."""
+    code (last_tile: the midpoint test that lets vanishing probabilities pass, which the last tile
+    and pieces take; else the cheaper one of the streaming blocks' tiles before; the bytes are the
+    same)."""
     dev = _require_device(x)
     x = x.float().contiguous()
     y = torch.empty(x.shape, dtype=torch.uint8, device=dev)

@@ -860,9 +860,9 @@ def _f32_bits(lo, hi):
 @pytest.mark.parametrize("last_tile", [False, True])
 def test_control_probability_bytes_exhaustive(last_tile):
     # Every binary32 input of the control path's P byte (x <= 8.8125 = the offset maximum 8.807
-    # plus its rounding): E4M3(RN_f32(exp2(x))) from the fused kernel's device function vs the
-    # oracle (binary64 exp2 rechecked in binary128), all 4.7e8 inputs with 2^-24 <= |x| <= 11 /
-    # 8.8125. Outside that range the byte is fixed: 1.0 (0x38) for |x| < 2^-24, 0 for x < -11.
+    # plus its rounding): E4M3(RN_f32(exp2(x))) from the fused kernel's device functions (both
+    # forms of its midpoint test, the byte that passes it, the recheck of one that does not) vs the
+    # oracle (binary64 exp2 rechecked in binary128), all 4.7e8 inputs with 2^-24 <= |x| <= 11 / 8.8125. Outside that range the byte is fixed: 1.0 (0x38) for |x| < 2^-24, 0 for x < -11.
     chunk = 1 << 25
     mism = 0
     for lo, hi in ((2.0 ** -24, 8.8125), (-(2.0 ** -24), -11.0)):
