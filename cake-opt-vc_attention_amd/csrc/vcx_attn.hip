@@ -178,7 +178,9 @@ __device__ __forceinline__ void attn_block(const AttnArgs& a, int64_t bh, int64_
   w.wide = 0;
   if constexpr (PM == 0) {
     // the cheap midpoint test until a vanishing probability; after an early end the rest
-    if constexpr (W::kCheapTest) body_tiles<true>(w, ld, a, t, lds0, lds1, meta0, meta1);
+    if constexpr (W::kCheapTest) {
+      if (!w.wide_scores(a)) body_tiles<true>(w, ld, a, t, lds0, lds1, meta0, meta1);
+    }
     body_tiles<false>(w, ld, a, t, lds0, lds1, meta0, meta1);
   } else if constexpr (PM == 2 && QF == 0) {
     if (w.fold_ok) body_tiles<true>(w, ld, a, t, lds0, lds1, meta0, meta1);

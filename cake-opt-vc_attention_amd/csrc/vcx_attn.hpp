@@ -515,6 +515,25 @@ struct Wave {
     }
   }
 
+  // Control path: whether probabilities of this wave's rows are likely to vanish, by the scales
+  // alone: the score (in bits) of a row and a key of the first tile whose entries are all their
+  // group's largest. N(0,1) inputs give 19 (D64) to 21, and as much more as Q is scaled by; from about
+  // 14 times on some probability of almost every block vanishes in the first tiles, which such a wave
+  // would do twice before it leaves the copy with the cheap test (see bytes). Only the copy of the
+  // tile loop depends on it, not a result. Same box, us, both neighbours' bytes of every probability /
+  // leaving alone / this, Q scaled by 1, 14 and 25: [1,32,2048 x 512,128] 27.7 / 24.9 / 24.9, 25.4 / 27.8 /
+  // 25.7, 25.1 / 28.4 / 22.9; [1,32,2048 x 1024,64] 33.2 / 29.4 / 29.7, 32.4 / 31.2 / 30.7, 32.5 / 34.3 / 29.7;
+  // [1,16,3000,128] with smoothing 97.2 / 87.4 / 87.5, 92.9 / 95.2 / 90.4, 93.0 / 91.2 / 86.5;
+  // [1,28,8192,128] 729 / 661 / 656, 698 / 667 / 655, 697 / 650 / 632.
+  __device__ inline bool wide_scores(const AttnArgs& a) const {
+    constexpr float kWide = 280.0f, kMax = QF == 1 ? 448.0f : 127.0f, kRootD = D == 128 ? 11.313708f : 8.0f;
+    const float ks0 = a.ks[QF == 1 ? bh_ * a.tiles : bh_ * a.tiles * 4 + G];
+    bool any = false;
+#pragma unroll
+    for (int qg = 0; qg < NQG; ++qg) any |= row[qg] < a.Nq && qsv[qg] * ks0 * a.sm * (kMax * kMax * kRootD) > kWide;
+    return wave_any(any);
+  }
+
   // Phase 3 of a tile for row group qg: the P bytes against the running maximum mx (and on
   // the control path the row's unrounded mass tmq).
   template <bool LAST, bool PRE>
@@ -578,10 +597,9 @@ struct Wave {
       // A vanishing probability (a score more than about 103 nats below the row maximum) always
       // fails the test: PRE takes none into account but sets wide, upon which the wave leaves for
       // the copy of the loop that lifts small probabilities over it, one more instruction per
-      // probability. Same box, us, both neighbours' bytes of every probability / lifted / this:
-      // smoothing [1,7,37741,128] 3830 / 3703 / 3528, [1,8,16000,64] 696 / 638 / 601, [1,16,3000,128]
-      // 94.4 / 92.1 / 87.3. With Q scaled by 25, where every wave leaves after its first two
-      // tiles: 3674 / 3460 / 3513, 689 / 627 / 648, 88.6 / 85.5 / 91.7.
+      // probability; a wave whose scales let it expect one (wide_scores) starts there. Same box, us,
+      // both neighbours' bytes of every probability / lifted / this: smoothing [1,7,37741,128] 3830 /
+      // 3703 / 3528, [1,8,16000,64] 696 / 638 / 601, [1,16,3000,128] 94.4 / 92.1 / 87.3.
       const float f = scl;
       float ls = -0.0f;  // -0 + p = p: the first addition folds away
       constexpr int kSpan = D == 128 ? 8 : 1;
