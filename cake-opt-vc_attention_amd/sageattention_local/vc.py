@@ -12,8 +12,8 @@ Differences a caller can observe, all deliberate:
 * Any current HIP stream is accepted (the reference required the default
   stream because an upstream kernel used it); all work is enqueued on it.
 * ``kernel_mode`` accepts the reference's documented mode names with the same
-  compatibility rules. Every mode runs the single gfx950 kernel (the names
-  select Hopper WGMMA/TMA schedules that have no MI355X counterpart); the
+  compatibility rules. The names select Hopper WGMMA/TMA schedules that have no
+  MI355X counterpart and choose no kernel here (the shape does); the
   numerics follow the mode as in the reference: without block values the
   default and vc12..vc15 modes use the folded ExpCast encode, vc4..vc11 the
   unfused one (``AFFINE_MODES``).
@@ -211,7 +211,7 @@ def sageattn_vc(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, re
 
 # The reference's kernel_resources names (vc_sm90.cu:801-808,1123-1213 and vc.py:113-118), each
 # mapped to the (value mode, probability mode) of the gfx950 kernel this module launches for
-# that mode at D128: value mode 0 = no block values, 1 = block values with channel scales;
+# that mode at D128 where the rows fill the chip: value mode 0 = no block values, 1 = block values with channel scales;
 # probability mode 0 = Sage FP8 control, 1 = unfused ExpCast, 2 = folded ExpCast
 # (AFFINE_MODES without block values). "smooth_*" / "full_*" are the reference's
 # block-value kernels without / with ExpCast; the sage-layout and vc31/vc32 entries follow
@@ -240,7 +240,9 @@ def kernel_resources(output_type=1):
     """Compiled resources per kernel mode under the reference's names (vc.py:113-118,
     vc_sm90.cu:786-822): registers_per_thread, local_bytes_per_thread (spill),
     static/dynamic_shared_bytes, threads_per_block, predicted_active_blocks_per_sm
-    (per CU here). Each name reports the gfx950 kernel this module runs for that mode."""
+    (per CU here). Each name reports the gfx950 kernel whose blocks stream every key tile
+    for that mode; a call of few rows runs as split pieces instead, whose 512-thread kernel
+    has no entry (piece_groups in csrc/vcx_attn_piece.hip)."""
     if output_type not in (0, 1) or isinstance(output_type, bool):
         raise RuntimeError("Output type must be 0 (FP16) or 1 (BF16)")
     ext = _extension()

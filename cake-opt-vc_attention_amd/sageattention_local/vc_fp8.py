@@ -65,7 +65,8 @@ def sageattn_vc_fp8(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None
 
 def fp8_kernel_resources(output_type=1, dim=128):
     """Compiled resources of the FP8 kernels (reference vc_fp8_kernel_resources,
-    fp8_dispatch.cuh:61-73): {"fp8_control": {...}, "fp8_expcast": {...}}."""
+    fp8_dispatch.cuh:61-73): {"fp8_control": {...}, "fp8_expcast": {...}}, of the streaming
+    blocks as in kernel_resources."""
     if output_type not in (0, 1) or dim not in (64, 128):
         raise ValueError("Expected output_type=0/1, D=64/128")
     ext = _extension()

@@ -598,7 +598,7 @@ def clock_probe(window_us: int, device=None) -> ClockProbe:
 
 
 def kernel_resources_mode(D: int, value_mode: int, expcast: int, output_type: int = 1) -> dict:
-    """Compiled resources of the fused kernel one launch mode runs (value_mode 0: no block
+    """Compiled resources of the streaming fused kernel of one launch mode (value_mode 0: no block
     values, 1: block values with channel scales, 2: per-block scales; expcast 0 control,
     1 unfused ExpCast, 2 folded), in the reference's key names (vc_sm90.cu:786-797)."""
     arr = (ctypes.c_int64 * 7)()

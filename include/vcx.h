@@ -275,14 +275,16 @@ int vcx_fp8_exp2_codes(const float* x, uint8_t* y, int64_t n, int form, void* st
  * parity tests to pin the instructions' rounding against the CPU oracle. */
 int vcx_convert_probe(const float* x, uint8_t* u8, uint8_t* f8, int64_t n, void* stream);
 
-/* Compiled resources of the fused kernel for (D, block_values):
+/* Compiled resources of the fused kernel whose blocks stream every key tile (what a call runs
+ * whose rows fill the chip; calls of few rows run split pieces, whose resources no entry
+ * reports) for (D, block_values):
  * out[0] VGPRs, out[1] AGPRs (0 if not reported), out[2] static LDS bytes,
  * out[3] dynamic LDS bytes per block, out[4] threads per block,
  * out[5] scratch (spill) bytes per lane.
  * Replaces _vc_sm90.kernel_resources (third_party/sageattention_local/csrc/vc/vc_sm90.cu:786-822). */
 int vcx_kernel_resources(int64_t D, int block_values, int64_t* out);
 
-/* Compiled resources of the fused kernel that one launch mode runs: value_mode 0 (no
+/* Compiled resources of the streaming fused kernel of one launch mode: value_mode 0 (no
  * block values), 1 (block values, channel scales), 2 (block values, per-block scales);
  * expcast 0/1/2 as for vcx_attention_fwd (2 only with value_mode 0); out_dtype
  * VCX_FLOAT16 / VCX_BFLOAT16. out[0..5] as for vcx_kernel_resources, out[6] the
