@@ -260,17 +260,24 @@ __device__ inline float row_xor(float v) {
 }
 
 // One butterfly stage of the rotation across lanes l and l ^ M: the lower entry becomes
-// RN(a + b), the upper one RN(a - b). The upper lane adds its own entry negated. With eight
-// entries per lane the DPP moves of one entry fill the wait states of another (rotated Q/K
-// quantization at [1,28,37741,128] 259 -> 228 us); with fewer they stall, and distances 4 and 8
-// take the LDS-pipe permute ([1,40,32760,64]: 159 us by DPP, 152 us so).
+// RN(a + b), the upper one RN(a - b). With eight entries per lane the upper lane adds its own entry
+// negated, and the DPP moves of one entry fill the wait states of another (rotated Q/K quantization at
+// [1,28,37741,128] 259 -> 228 us). With fewer they stall: distances 4 and 8 take the LDS-pipe permute
+// ([1,40,32760,64]: 159 us by DPP, 152 us so), and a select between sum and difference is shorter than
+// the negation before the move ([1,2,2048,64] fp16 12.0 -> 10.9 us, [1,28,20000,64] bf16 72 -> 69 us).
 template <int M, int CPT>
 __device__ inline void hadamard_lanes(float (&x)[CPT], int c) {
-  const uint32_t flip = (c & M) ? 0x80000000u : 0u;
+  if constexpr (CPT < 8) {
 #pragma unroll
-  for (int j = 0; j < CPT; ++j)
-    x[j] = __fadd_rn(M >= 4 && CPT < 8 ? __shfl_xor(x[j], M, 64) : row_xor<M>(x[j]),
-                     __uint_as_float(__float_as_uint(x[j]) ^ flip));
+    for (int j = 0; j < CPT; ++j) {
+      const float other = M >= 4 ? __shfl_xor(x[j], M, 64) : row_xor<M>(x[j]);
+      x[j] = (c & M) ? __fsub_rn(other, x[j]) : __fadd_rn(x[j], other);
+    }
+  } else {
+    const uint32_t flip = (c & M) ? 0x80000000u : 0u;
+#pragma unroll
+    for (int j = 0; j < CPT; ++j) x[j] = __fadd_rn(row_xor<M>(x[j]), __uint_as_float(__float_as_uint(x[j]) ^ flip));
+  }
 }
 
 // One butterfly stage between a lane's entries j and j + S.
