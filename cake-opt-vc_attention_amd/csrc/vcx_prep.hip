@@ -130,7 +130,19 @@ __device__ __forceinline__ void tile_stats_body(const Strided& t, int64_t H, int
   // statistics read them twice, and packed they take half the registers
   Row<D> rows[8];
   load_key_rows_packed<D, 8>(base, sn, perm, bh, n, tile * kTile + kk, c, rows);
-  auto v = [&](int i, int j) -> float { return tile * kTile + kk + 16 * i < n ? row_val<DT, D>(rows[i], j) : 0.0f; };
+  // Keys past n, which only the last tile has, read as zero. The smoothing statistics, which read
+  // every value twice, clear the packed rows of such a tile and spare the others the selects
+  // ([1,28,20000,64] fp16 prepare_v with block scales 42.2 -> 39.1 us); one pass is shorter with them.
+  const bool full = (tile + 1) * kTile <= n;
+  if (MODE == kVSmooth && !full) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+#pragma unroll
+      for (int k = 0; k < CPT / 2; ++k) rows[i].w[k] = tile * kTile + kk + 16 * i < n ? rows[i].w[k] : 0u;
+  }
+  auto v = [&](int i, int j) -> float {
+    return MODE == kVSmooth || tile * kTile + kk + 16 * i < n ? row_val<DT, D>(rows[i], j) : 0.0f;
+  };
   const int64_t meta = (bh * tiles + tile) * D;
   if constexpr (MODE == kVAmax) {
     float m[CPT];
@@ -174,15 +186,21 @@ __device__ __forceinline__ void tile_stats_body(const Strided& t, int64_t H, int
 #pragma unroll
         for (int k = 0; k < CPT / 2; ++k) asm volatile("" : "+v"(rows[i].w[k]));
       float pk[CPT];
+      auto peaks = [&](auto masked) {
 #pragma unroll
-      for (int j = 0; j < CPT; ++j) {
-        float mu = mean_sh[c * CPT + j];
-        pk[j] = 0.0f;
+        for (int j = 0; j < CPT; ++j) {
+          float mu = mean_sh[c * CPT + j];
+          pk[j] = 0.0f;
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (tile * kTile + kk + 16 * i < n) pk[j] = fmaxf(pk[j], fabsf(__fsub_rn(v(i, j), mu)));
-        pk[j] = max_xor32(max_xor16(pk[j]));
-      }
+          for (int i = 0; i < 8; ++i)
+            if (!decltype(masked)::value || tile * kTile + kk + 16 * i < n)
+              pk[j] = fmaxf(pk[j], fabsf(__fsub_rn(v(i, j), mu)));
+        }
+      };
+      if (full) peaks(std::false_type());
+      else peaks(std::true_type());
+#pragma unroll
+      for (int j = 0; j < CPT; ++j) pk[j] = max_xor32(max_xor16(pk[j]));
       if (lane < 16)
 #pragma unroll
         for (int j = 0; j < CPT; ++j) fred[w * D + c * CPT + j] = pk[j];
