@@ -205,7 +205,7 @@ def sageattn_vc(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None, re
     _extension().attention_call(q, k, v, out, expcast=_encode(expcast, v_smooth, kernel_mode), smooth=v_smooth,
                                 channel_scale=v_scale_mode == "channel", clusters=clusters, iterations=iterations,
                                 legacy=grouping_mode == "legacy",
-                                scale=q.shape[-1] ** -0.5 if sm_scale is None else sm_scale)
+                                scale=q.shape[-1] ** -0.5 if sm_scale is None else sm_scale, validated=True)
     return result
 
 

@@ -59,7 +59,7 @@ def sageattn_vc_fp8(q, k, v, tensor_layout="HND", is_causal=False, sm_scale=None
     if tensor_layout == "NHD":
         q, k, v, out = (x.transpose(1, 2) for x in (q, k, v, out))  # strided HND views, no copy
     _extension().attention_call(q, k, v, out, qk_fp8=True, expcast=2 if expcast else 0, smooth=False,
-                                scale=q.shape[-1] ** -0.5 if sm_scale is None else sm_scale)
+                                scale=q.shape[-1] ** -0.5 if sm_scale is None else sm_scale, validated=True)
     return result
 
 

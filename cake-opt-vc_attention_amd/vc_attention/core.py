@@ -231,7 +231,8 @@ def attention(q, k, v, config=None, *, cache=None, step=0, total_steps=1, reques
     # The ExpCast encode of the reference's default kernel mode: folded without block values.
     out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
     vcx.attention_call(q, k, v, out, perm=pi, rotate=cfg.qk_hadamard,
-                       expcast=(1 if active else 2) if cfg.expcast else 0, smooth=active, scale=scale)
+                       expcast=(1 if active else 2) if cfg.expcast else 0, smooth=active, scale=scale,
+                       validated=True)
     return out, {
         "backend": "hip",
         "smoothing_active": active,
